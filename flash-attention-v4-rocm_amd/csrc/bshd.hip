@@ -319,23 +319,41 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
 // with sq queries and sk keys sees keys j <= sk - sq + i).
 constexpr int BOTTOM_RIGHT = 2;
 
+// Up to this many items per resident workgroup, the packed kernel's lists go
+// by each q tile's own keys, else by its sequence's: with few rounds the last
+// items decide (4 x 2048 tokens H16 causal, 1 round: 77 us by tile, 97 by
+// sequence; 8 x 4096 H8, 4 rounds: 264 and 313), with many the q tiles of a
+// sequence profit from running together (32 x 1024..7168 H8, 8 rounds: 874 and
+// 844; 8 x 4096 H32, 16 rounds: 1092 and 1065).
+constexpr int BY_ITEM_ROUNDS = 4;
+
 template <int WAVES>
-void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int total, int grid, hipStream_t stream) {
-    const dim3 block(WAVES * 64);
+void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int total, hipStream_t stream) {
+    // One workgroup per item, in rows of MAX_GRID (a dimension is limited to 2^32 threads).
+    const int rows = int((total + MAX_GRID - 1) / MAX_GRID);
+    const dim3 grid(unsigned((total + rows - 1) / rows), unsigned(rows)), block(WAVES * 64);
+    int key_bits = 1;                          // of the longest sequence's key tile count
+    while (((a.max_seqlen_k + 63) / 64) >> key_bits) ++key_bits;
+    const int slots = device_cus() * 8 / WAVES;            // workgroups resident at once
+    const bool by_item = total <= BY_ITEM_ROUNDS * slots;
     if (causal == BOTTOM_RIGHT && a.lse)
-        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, true, WAVES, true>), dim3(grid), block, 0, stream, a,
-                           tiles, total);
+        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, true, WAVES, true>), grid, block, 0, stream, a,
+                           tiles, total, key_bits, by_item);
     else if (causal == BOTTOM_RIGHT)
-        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, false, WAVES, true>), dim3(grid), block, 0, stream, a,
-                           tiles, total);
+        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, false, WAVES, true>), grid, block, 0, stream, a,
+                           tiles, total, key_bits, by_item);
     else if (causal && a.lse)
-        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, true, WAVES>), dim3(grid), block, 0, stream, a, tiles, total);
+        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, true, WAVES>), grid, block, 0, stream, a, tiles, total,
+                           key_bits, by_item);
     else if (causal)
-        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, false, WAVES>), dim3(grid), block, 0, stream, a, tiles, total);
+        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, false, WAVES>), grid, block, 0, stream, a, tiles, total,
+                           key_bits, by_item);
     else if (a.lse)
-        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, false, true, WAVES>), dim3(grid), block, 0, stream, a, tiles, total);
+        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, false, true, WAVES>), grid, block, 0, stream, a, tiles, total,
+                           key_bits, by_item);
     else
-        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, false, false, WAVES>), dim3(grid), block, 0, stream, a, tiles, total);
+        hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, false, false, WAVES>), grid, block, 0, stream, a, tiles, total,
+                           key_bits, by_item);
 }
 
 // Checks of the packed-sequence arguments (before any HIP call); the shape
@@ -580,13 +598,16 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_varlen(c
     const bool small = a->max_seqlen_q <= 1024 || int64_t(a->batch) * a->heads * tiles256 < device_cus();
     const int bm = small ? 128 : 256;
     const int tiles = (a->max_seqlen_q + bm - 1) / bm;
-    const int64_t total = int64_t(a->batch) * a->heads * tiles;
+    int64_t total = int64_t(a->batch) * a->heads * tiles;
     if (total > INT_MAX) return hipErrorInvalidValue;
-    const int grid = int(total < MAX_GRID ? total : MAX_GRID);
+    // The sorted item lists hold only the q tiles that exist, and no batch of
+    // total_q rows has more than this many of them.
+    if (a->batch <= fav4::MAX_SORTED_SEQS)
+        total = std::min(total, a->heads * ((a->total_q + int64_t(a->batch) * (bm - 1)) / bm));
     if (small)
-        launch_varlen<4>(*a, causal, tiles, int(total), grid, stream);
+        launch_varlen<4>(*a, causal, tiles, int(total), stream);
     else
-        launch_varlen<8>(*a, causal, tiles, int(total), grid, stream);
+        launch_varlen<8>(*a, causal, tiles, int(total), stream);
     return hipGetLastError();
 }
 

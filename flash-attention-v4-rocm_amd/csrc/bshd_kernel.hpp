@@ -28,6 +28,8 @@
 #include "fav4_bshd.h"
 #include "gfx950.hpp"
 
+#include <climits>
+
 namespace fav4 {
 
 constexpr int D = 128;
@@ -67,6 +69,90 @@ __device__ __forceinline__ void for_each_item(int tiles, int total, F&& process)
         } else {
             process(bh, j);
         }
+    }
+}
+
+// Query rows [qs, qe) and keys [ks, ke) of one packed sequence.
+struct Span {
+    int qs, qe, ks, ke;
+};
+
+// Work items of a packed batch, taken from the sequences' lengths on the
+// device.  One head's items are ranked by descending weight, equal weights by
+// sequence: a ragged batch starts its long items first and ends on its
+// shortest, and nothing is launched for the q tiles that a shorter sequence
+// does not have.  A sequence has `tiles` items; those that weigh c or more are
+// all of them while (c - 1) * UNIT < keys, less one for every BM by which
+// (c - 1) * UNIT passes `shift` (c = 0: all).  Each wave finds item `rank` by itself, the
+// sequences (up to 4 * 64) in its lanes: a binary search for the weight, of
+// key_bits bits, whose items hold `rank`, then one scan over the sequences
+// (some 200 instructions, about 0.6 us against 8 us and more for an item).
+// Returns the sequence, its span and the item's place among that sequence's
+// (0 = its heaviest); seq = -1 past the last item.
+constexpr int MAX_SORTED_SEQS = 256;
+struct PackedSeq {
+    Span span;
+    int tiles, keys, shift;
+};
+struct PackedItem {
+    int seq, place;
+    Span span;
+};
+template <int REGS, int BM, int UNIT, class Load>
+__device__ __forceinline__ PackedItem sorted_item_in(int rank, int batch, int key_bits, int lane, Load&& load) {
+    PackedSeq s[REGS];                         // sequence 64 * k + lane
+#pragma unroll
+    for (int k = 0; k < REGS; ++k) {
+        s[k] = load(min(k * 64 + lane, batch - 1));
+        if (k * 64 + lane >= batch) s[k].tiles = 0;
+    }
+    auto at_least = [&](int k, int c) {
+        const int below = (c - 1) * UNIT;
+        if (c == 0) return s[k].tiles;         // those without a visible key too
+        return s[k].keys > below ? max(0, s[k].tiles - max(0, below - s[k].shift) / BM) : 0;
+    };
+    int c = 0, above = 0;                      // weight so far; items that weigh more
+    for (int bit = 1 << (key_bits - 1); bit; bit >>= 1) {
+        int n = 0;
+#pragma unroll
+        for (int k = 0; k < REGS; ++k) n += at_least(k, c + bit);
+        n = wave_total(n);
+        if (n > rank) c += bit;
+        else above = n;
+    }
+    int r = rank - above;
+#pragma unroll
+    for (int k = 0; k < REGS; ++k) {
+        const int before = at_least(k, c + 1), mine = at_least(k, c) - before, end = wave_scan(mine);
+        const uint64_t hit = __builtin_amdgcn_ballot_w64(end > r);
+        if (hit) {
+            const int l = __builtin_ctzll(hit);
+            auto at = [&](int x) { return __builtin_amdgcn_readlane(x, l); };
+            return {k * 64 + l, r - at(end - mine - before),
+                    {at(s[k].span.qs), at(s[k].span.qe), at(s[k].span.ks), at(s[k].span.ke)}};
+        }
+        r -= __builtin_amdgcn_readlane(end, 63);
+    }
+    return {-1, 0, {}};
+}
+template <int BM, int UNIT, class Load>
+__device__ __forceinline__ PackedItem sorted_item(int rank, int batch, int key_bits, int lane, Load&& load) {
+    return batch <= 64 ? sorted_item_in<1, BM, UNIT>(rank, batch, key_bits, lane, load)
+                       : sorted_item_in<MAX_SORTED_SEQS / 64, BM, UNIT>(rank, batch, key_bits, lane, load);
+}
+
+// Item id -> (head, rank in the head's item list).  heads a multiple of 8:
+// each XCD (id % 8) works on heads/8 heads, taking their equal ranks side by
+// side, so the query heads of a K/V head share its keys in that XCD's L2;
+// else the heads are dealt round-robin.
+__device__ __forceinline__ void packed_head_rank(int id, int heads, int& head, int& rank) {
+    if ((heads & 7) == 0) {
+        const int per = heads >> 3, slot = id >> 3;
+        rank = slot / per;
+        head = (id & 7) * per + slot - rank * per;
+    } else {
+        rank = id / heads;
+        head = id - rank * heads;
     }
 }
 
@@ -988,7 +1074,7 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
 // ---------------------------------------------------------------------------
 template <int BN, bool CAUSAL, bool LSE, int WAVES, bool BR = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total) {
+void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, bool by_item) {
     static_assert(!BR || CAUSAL, "bottom-right is a causal mask");
     constexpr int BM = WAVES * 32;
     constexpr int TILE_BYTES = BN * ROW_BYTES;
@@ -1010,37 +1096,78 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total) {
     const LdsOffsets off = lds_offsets(lane);
     const DmaOffsets<DMA> dofs = dma_offsets<DMA>(wave, lane, kv_row_bytes, kv_row_bytes);
 
-    // Item order.  Each XCD gets a contiguous run of logical items (all q
+    // A sequence's query rows and keys, clamped as described above.
+    auto span = [&](int b) {
+        const int qs = min(max(a.cu_seqlens_q[b], 0), a.total_q);
+        const int qe = min(max(a.cu_seqlens_q[b + 1], qs), min(a.total_q, qs + a.max_seqlen_q));
+        const int ks = min(max(a.cu_seqlens_k[b], 0), a.total_k);
+        const int ke = min(max(a.cu_seqlens_k[b + 1], ks), min(a.total_k, ks + a.max_seqlen_k));
+        return Span{qs, qe, ks, ke};
+    };
+    // Item order, up to MAX_SORTED_SEQS sequences: sorted_item's lists.  A q
+    // tile weighs its key tiles (by_item: with few items per workgroup slot,
+    // where the last ones decide) or its sequence's longest tile's (its q
+    // tiles then run together, heaviest first, and share its K/V in L2).
+    // Against the order below (graph-timed, causal): 24 sequences of 64..4096
+    // tokens H32 KVH8 708 -> 582 us, 64 of 100..1000 H8 69 -> 55, 4 x 2048
+    // H16 105 -> 77 (by sequence 97), 8 x 4096 H8 313 -> 264 (313); 32 of
+    // 1024..7168 H8 858 -> 848.
+    // Larger batches: each XCD gets a contiguous run of logical items (all q
     // tiles of a (sequence, head) together, for its L2), but the runs are cut
     // from the (sequence, head) pairs taken column by column from an 8-wide
     // grid, bh = 8*row + col: XCD x holds mostly the pairs with bh % 8 == x,
     // i.e. a share of every sequence rather than a few whole sequences, so
     // ragged lengths do not leave XCDs idle.  Within a pair the q tiles run
     // last-to-first (causal: heaviest first).
+    const bool sorted = a.batch <= MAX_SORTED_SEQS;
     const int nbh = a.batch * a.heads, full = nbh >> 3, rem8 = nbh & 7;
-    for (int id = blockIdx.x; id < total; id += gridDim.x) {
-        const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
-        const int logical = xcd * per + min(xcd, rem) + slot;
-        const int j = __builtin_amdgcn_readfirstlane(logical / tiles);
-        const int tile = __builtin_amdgcn_readfirstlane(tiles - 1 - (logical - j * tiles));
-        int gcol, grow;
-        if (j < rem8 * (full + 1)) {
-            gcol = j / (full + 1);
-            grow = j - gcol * (full + 1);
+    {
+        // One item per workgroup (no loop over items: the state it would keep
+        // live through the key loop costs that loop its V reads' depth).
+        const int id = int(blockIdx.y * gridDim.x + blockIdx.x);
+        if (id >= total) return;
+        int batch, head, tile;
+        Span sp;
+        if (sorted) {
+            int rank;
+            packed_head_rank(id, a.heads, head, rank);
+            const PackedItem it = sorted_item<BM, BN>(rank, a.batch, key_bits, lane, [&](int b) {
+                // A q tile's visible keys reach the diagonal of its last row.
+                const Span s = span(b);
+                const int nq = s.qe - s.qs, nk = s.ke - s.ks;
+                return PackedSeq{s, (nq + BM - 1) / BM, CAUSAL && !BR ? min(nq, nk) : nk,
+                                 !CAUSAL || !by_item ? INT_MAX : BR ? nk - nq : 0};
+            });
+            if (it.seq < 0) return;
+            batch = it.seq;
+            sp = it.span;
+            tile = (sp.qe - sp.qs + BM - 1) / BM - 1 - it.place;       // from the last q tile down
         } else {
-            const int jj = j - rem8 * (full + 1);
-            gcol = rem8 + jj / full;
-            grow = jj - (gcol - rem8) * full;
+            const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
+            const int logical = xcd * per + min(xcd, rem) + slot;
+            const int j = __builtin_amdgcn_readfirstlane(logical / tiles);
+            tile = __builtin_amdgcn_readfirstlane(tiles - 1 - (logical - j * tiles));
+            int gcol, grow;
+            if (j < rem8 * (full + 1)) {
+                gcol = j / (full + 1);
+                grow = j - gcol * (full + 1);
+            } else {
+                const int jj = j - rem8 * (full + 1);
+                gcol = rem8 + jj / full;
+                grow = jj - (gcol - rem8) * full;
+            }
+            const int bh = grow * 8 + gcol;
+            batch = bh / a.heads;
+            head = bh - batch * a.heads;
+            sp = span(batch);
         }
-        const int bh = grow * 8 + gcol;
-        const int batch = bh / a.heads, head = bh - batch * a.heads;
-        const int qs = min(max(__builtin_amdgcn_readfirstlane(a.cu_seqlens_q[batch]), 0), a.total_q);
-        const int qe = min(max(__builtin_amdgcn_readfirstlane(a.cu_seqlens_q[batch + 1]), qs), min(a.total_q, qs + a.max_seqlen_q));
-        const int ks = min(max(__builtin_amdgcn_readfirstlane(a.cu_seqlens_k[batch]), 0), a.total_k);
-        const int ke = min(max(__builtin_amdgcn_readfirstlane(a.cu_seqlens_k[batch + 1]), ks), min(a.total_k, ks + a.max_seqlen_k));
-        const int sq = qe - qs, sk = ke - ks;
+        batch = __builtin_amdgcn_readfirstlane(batch);
+        head = __builtin_amdgcn_readfirstlane(head);
+        tile = __builtin_amdgcn_readfirstlane(tile);
+        const int qs = __builtin_amdgcn_readfirstlane(sp.qs), ks = __builtin_amdgcn_readfirstlane(sp.ks);
+        const int sq = __builtin_amdgcn_readfirstlane(sp.qe) - qs, sk = __builtin_amdgcn_readfirstlane(sp.ke) - ks;
         const int q0 = tile * BM;
-        if (q0 >= sq) continue;    // uniform over the workgroup
+        if (q0 >= sq) return;    // uniform over the workgroup
         const int qw = q0 + wave * 32, row = qw + col;
         const int64_t qrow0 = (int64_t(qs) + q0) * a.heads + head;
         const int64_t krow0 = int64_t(ks) * a.kv_heads + head / group;
@@ -1137,8 +1264,6 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total) {
         if constexpr (LSE) {
             if (half == 0 && row < sq) a.lse[int64_t(head) * a.total_q + qs + row] = __builtin_fmaf(st.m, LN2, logf(st.l));
         }
-        wait_vmem();
-        __syncthreads();
     }
 }
 

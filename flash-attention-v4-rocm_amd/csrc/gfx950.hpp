@@ -131,6 +131,20 @@ __device__ __forceinline__ float xhalf_sum(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Inclusive sum over the wave's lanes 0..l (DPP shifts inside the 16-lane rows,
+// then the rows' last lanes broadcast forward); every lane must be active.
+// Lane 63 holds the wave's total.
+__device__ __forceinline__ int wave_scan(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);   // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);   // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);   // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+    return x;
+}
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+
 __device__ __forceinline__ float exp2_native(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // acc + x.lo + x.hi in FP32 (v_dot2c_f32_bf16 against the pair (1, 1)).

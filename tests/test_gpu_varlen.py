@@ -205,3 +205,51 @@ def test_varlen_bottom_right_causal(gpu_runner, case):
         if sq == sk and sq > 0:
             assert torch.equal(o[a:b].view(torch.int16), o_tl[a:b].view(torch.int16)), i
             assert torch.equal(lse[:, a:b].view(torch.int32), lse_tl[:, a:b].view(torch.int32)), i
+
+
+# (heads, kv_heads, sequences, longest): batches at the edges of the item
+# lists (one, and either side of 64 and of 256 sequences), heads in whole
+# XCD shares and not, few items per workgroup slot and many, both tile sizes.
+LIST_CASES = [(1, 1, 1, 300), (3, 1, 63, 300), (8, 8, 64, 130), (16, 2, 65, 700), (8, 2, 255, 260), (16, 4, 256, 300),
+              (5, 5, 257, 200), (32, 4, 40, 1300)]
+
+
+@pytest.mark.parametrize("case", LIST_CASES, ids=lambda c: "h%dkv%d_n%d_max%d" % c)
+def test_varlen_item_lists(gpu_runner, case):
+    """Every (sequence, head, q tile) is attended once: each sequence's rows
+    bitwise those of a call on that sequence alone, for the three masks, with
+    empty sequences and query counts on both sides of the tile edges."""
+    import torch
+    h, kvh, n, longest = case
+    rng = np.random.default_rng(n * 1000 + h)
+    sq = rng.integers(0, longest + 1, n)
+    sk = rng.integers(0, longest + 1, n)
+    edges = np.array([0, 1, 127, 128, 129, 255, 256, 257, longest])
+    sq[:edges.size] = np.minimum(edges, longest)[:n]
+    sk[-1] = sq[-1] = longest
+    cu_q, cu_k = (np.concatenate([[0], np.cumsum(x)]).astype(np.int32) for x in (sq, sk))
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(n)
+    make = lambda rows, heads: torch.randn((rows, heads, 128), generator=gen, device=dev).to(torch.bfloat16)
+    q, k, v = make(int(cu_q[-1]), h), make(int(cu_k[-1]), kvh), make(int(cu_k[-1]), kvh)
+    for causal in (0, 1, 2):
+        print(f"  lists h{h} kv{kvh} n{n} causal {causal}", flush=True)
+        o, lse, og, lg = _run_varlen(gpu_runner, q, k, v, cu_q, cu_k, longest, longest, causal, True)
+        assert torch.isnan(og).all().item() and torch.isnan(lg).all().item()
+        for i in range(n):
+            a, b, c, d = int(cu_q[i]), int(cu_q[i + 1]), int(cu_k[i]), int(cu_k[i + 1])
+            if a == b:
+                continue
+            if c == d:
+                assert (o[a:b] == 0).all().item() and (lse[:, a:b] == float("-inf")).all().item(), i
+                continue
+            o_ref = torch.full((1, b - a, h, 128), float("nan"), device=dev, dtype=torch.bfloat16)
+            l_ref = torch.full((1, h, b - a), float("nan"), device=dev, dtype=torch.float32)
+            if causal == 2:
+                one = lambda x: torch.tensor([0, x], device=dev, dtype=torch.int32)
+                gpu_runner.call_varlen(q[a:b], k[c:d], v[c:d], o_ref[0], l_ref[0], one(b - a), one(d - c), b - a,
+                                       d - c, 2)
+            else:
+                gpu_runner.call_gqa(q[None, a:b], k[None, c:d], v[None, c:d], o_ref, l_ref, causal, 2)
+            assert torch.equal(o[a:b].view(torch.int16), o_ref[0].view(torch.int16)), (causal, i, b - a, d - c)
+            assert torch.equal(lse[:, a:b].view(torch.int32), l_ref[0].view(torch.int32)), (causal, i, b - a, d - c)
