@@ -17,19 +17,44 @@ namespace {
 // Upper bound on launched workgroups; larger problems loop inside the kernel.
 constexpr int64_t MAX_GRID = int64_t(1) << 22;
 
+// CU count of the current device (256 if it cannot be read), cached per
+// device after the first query.
+int device_cus() {
+    static std::atomic<int> cache[64];
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    const bool slot = dev >= 0 && dev < 64;
+    if (slot && (cus = cache[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+    if (slot) cache[dev].store(cus, std::memory_order_relaxed);
+    return cus;
+}
+
+// One workgroup per item, in rows of at most MAX_GRID (a grid dimension holds
+// fewer than 2^32 threads).
+dim3 item_grid(int64_t total) {
+    const int64_t rows = (total + MAX_GRID - 1) / MAX_GRID;
+    return dim3(unsigned((total + rows - 1) / rows), unsigned(rows));
+}
+
 template <int WAVES, int BN, int STAGES, bool PIPE, bool CAUSAL>
 int launch(const Fav4Args& a, const fav4::Layout& L, hipStream_t stream) {
     constexpr int BM = WAVES * 32;
     const int tiles = (a.sq + BM - 1) / BM;
-    const int64_t total = int64_t(fav4::items_per_head<CAUSAL>(tiles)) * a.batch * a.heads;
+    const int64_t bh = int64_t(a.batch) * a.heads;
+    // Causal q tiles go in pairs of equal cost unless each has a CU of its own
+    // (B3 H5 S1500, 180 q tiles: 33.8 us paired, 29.4 not; B4 H16 S2048, 1024
+    // q tiles: 82 and 113).
+    const bool paired = CAUSAL && bh * tiles > device_cus();
+    const int64_t total = bh * fav4::items_per_head(tiles, paired);
     if (total > INT_MAX) return hipErrorInvalidValue;
-    const int grid = int(total < MAX_GRID ? total : MAX_GRID);
+    const dim3 grid = item_grid(total);
     if (a.lse)
-        hipLaunchKernelGGL((fav4::fwd_kernel<WAVES, BN, CAUSAL, true, STAGES, PIPE>), dim3(grid),
-                           dim3(WAVES * 64), 0, stream, a, L, tiles, int(total));
+        hipLaunchKernelGGL((fav4::fwd_kernel<WAVES, BN, CAUSAL, true, STAGES, PIPE>), grid, dim3(WAVES * 64), 0,
+                           stream, a, L, tiles, int(total), paired);
     else
-        hipLaunchKernelGGL((fav4::fwd_kernel<WAVES, BN, CAUSAL, false, STAGES, PIPE>), dim3(grid),
-                           dim3(WAVES * 64), 0, stream, a, L, tiles, int(total));
+        hipLaunchKernelGGL((fav4::fwd_kernel<WAVES, BN, CAUSAL, false, STAGES, PIPE>), grid, dim3(WAVES * 64), 0,
+                           stream, a, L, tiles, int(total), paired);
     return hipGetLastError();
 }
 
@@ -109,19 +134,6 @@ struct SplitPlan {
     int tiles;         // q tiles per item
     int64_t items;     // (batch, head) items, or (batch, K/V head) groups for decode
 };
-
-// CU count of the current device (256 if it cannot be read), cached per
-// device after the first query.
-int device_cus() {
-    static std::atomic<int> cache[64];
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    const bool slot = dev >= 0 && dev < 64;
-    if (slot && (cus = cache[dev].load(std::memory_order_relaxed)) > 0) return cus;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-    if (slot) cache[dev].store(cus, std::memory_order_relaxed);
-    return cus;
-}
 
 // Auto for prefill (Sq > 32).  Filling the CUs is not enough: on the small
 // grids where splitting is considered, the unsplit forward runs 128-row q
@@ -329,9 +341,7 @@ constexpr int BY_ITEM_ROUNDS = 4;
 
 template <int WAVES>
 void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int total, hipStream_t stream) {
-    // One workgroup per item, in rows of MAX_GRID (a dimension is limited to 2^32 threads).
-    const int rows = int((total + MAX_GRID - 1) / MAX_GRID);
-    const dim3 grid(unsigned((total + rows - 1) / rows), unsigned(rows)), block(WAVES * 64);
+    const dim3 grid = item_grid(total), block(WAVES * 64);
     int key_bits = 1;                          // of the longest sequence's key tile count
     while (((a.max_seqlen_k + 63) / 64) >> key_bits) ++key_bits;
     const int slots = device_cus() * 8 / WAVES;            // workgroups resident at once

@@ -49,26 +49,34 @@ __device__ __forceinline__ int v_swz(int r) { return ((r & 3) << 2) | ((r >> 2) 
 // Work items.  The hardware deals workgroups round-robin over the 8 XCDs, so
 // item ids are remapped to give each XCD a contiguous run of items: all q
 // tiles of one (batch, head) then run at the same time on one XCD and share
-// its L2 copy of that head's K/V.  Dense: one item = one q tile.  Causal: one
-// item = the pair of q tiles (j, tiles-1-j), heavy one first, so every item
-// costs tiles+1 key tiles and the grid has no tail of light items.
-template <bool CAUSAL>
-__host__ __device__ constexpr int items_per_head(int tiles) { return CAUSAL ? (tiles + 1) / 2 : tiles; }
+// its L2 copy of that head's K/V.  Dense: one item = one q tile.  Causal,
+// paired: one item = the pair of q tiles (j, tiles-1-j), heavy one first, so
+// every item costs tiles+1 key tiles and the grid has no tail of light items;
+// unpaired (when every q tile has a CU of its own): one q tile, heavy first.
+// One item per workgroup: the state that a loop over items keeps live through
+// the key loop cost that loop 30 VGPRs and its operand reads' depth.
+__host__ __device__ constexpr int items_per_head(int tiles, bool paired) { return paired ? (tiles + 1) / 2 : tiles; }
 
 template <bool CAUSAL, class F>
-__device__ __forceinline__ void for_each_item(int tiles, int total, F&& process) {
-    const int per_head = items_per_head<CAUSAL>(tiles);
-    for (int id = blockIdx.x; id < total; id += gridDim.x) {
-        const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
-        const int logical = xcd * per + min(xcd, rem) + slot;
-        const int bh = __builtin_amdgcn_readfirstlane(logical / per_head);
-        const int j = __builtin_amdgcn_readfirstlane(logical - bh * per_head);
-        if constexpr (CAUSAL) {
-            const int n = (j == tiles - 1 - j) ? 1 : 2;
-            for (int k = 0; k < n; ++k) process(bh, k == 0 ? tiles - 1 - j : j);
-        } else {
-            process(bh, j);
+__device__ __forceinline__ void for_item(int tiles, int total, bool paired, F&& process) {
+    const int id = int(blockIdx.y * gridDim.x + blockIdx.x);
+    if (id >= total) return;
+    const int per_head = items_per_head(tiles, CAUSAL && paired);
+    const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
+    const int logical = xcd * per + min(xcd, rem) + slot;
+    const int bh = __builtin_amdgcn_readfirstlane(logical / per_head);
+    const int j = __builtin_amdgcn_readfirstlane(logical - bh * per_head);
+    if constexpr (CAUSAL) {
+        const int last = paired ? j : tiles - 1 - j;
+        for (int tile = tiles - 1 - j;; tile = last) {
+            process(bh, tile);
+            if (tile == last) break;
+            // Clamped prefetches and O stores have landed before the stages are reused.
+            wait_vmem();
+            __syncthreads();
         }
+    } else {
+        process(bh, j);
     }
 }
 
@@ -245,7 +253,13 @@ __device__ __forceinline__ void dma_tile(u32x4 rk, u32x4 rv, uint32_t stage, int
     dma_kv<DMA, NT>(rk, rv, stage, stage + TILE_BYTES, wave, d);
 }
 
-// S^T = K.Q^T for one tile: 8 MFMAs per 32-key block, K operands read ahead.
+// S^T = K.Q^T for one tile: 8 MFMAs per 32-key block, taken dim chunk by dim
+// chunk over the blocks, so that neighbouring MFMAs feed different
+// accumulators, with the K operands read two chunks ahead.  The scheduling
+// barriers hold that order: left alone, the compiler picks it or a chain per
+// block with the register pressure around it, and the chain is 2-4% slower
+// (packed 8 x 4096 H32 causal 1069 us against 1028; three or all eight chunks
+// ahead lose again on the dense forward).
 // Masked tiles compute every block too (no branch around blocks past the key
 // length or above the diagonal): tile_mask then hides them, and the tile
 // stays one basic block for the scheduler.  K rows past sk hold zeros (the
@@ -255,14 +269,20 @@ __device__ __forceinline__ void tile_qk(const unsigned char* ks, const LdsOffset
                                         f32x16 (&s)[BN / 32]) {
     constexpr int KB = BN / 32;
     const f32x16 zero = {};
+    bf16x8 kop[8][KB];
+    auto read = [&](int c) {
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-        bf16x8 kop[8];
+        for (int kb = 0; kb < KB; ++kb) kop[c][kb] = lds_read16(ks + kb * 32 * ROW_BYTES + off.k[c]);
+    };
+    read(0);
+    read(1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) kop[c] = lds_read16(ks + kb * 32 * ROW_BYTES + off.k[c]);
-        s[kb] = mfma32(kop[0], qr[0], zero);
+    for (int c = 0; c < 8; ++c) {
+        if (c + 2 < 8) read(c + 2);
 #pragma unroll
-        for (int c = 1; c < 8; ++c) s[kb] = mfma32(kop[c], qr[c], s[kb]);
+        for (int kb = 0; kb < KB; ++kb) s[kb] = mfma32(kop[c][kb], qr[c], c ? s[kb] : zero);
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -518,7 +538,7 @@ __device__ __forceinline__ void store_o_rows(const RowState& st, float inv, unsi
 // stage at 64 KiB or more would otherwise cost an address add per read).
 template <int WAVES, int BN, bool CAUSAL, bool LSE, int STAGES, bool PIPE = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void fwd_kernel(Fav4Args a, Layout L, int tiles, int total) {
+void fwd_kernel(Fav4Args a, Layout L, int tiles, int total, bool paired) {
     static_assert(PIPE ? STAGES == 3 : STAGES == 2, "two stages, or three with the cross-tile pipeline");
     constexpr int BM = WAVES * 32;
     constexpr int TILE_BYTES = BN * ROW_BYTES;
@@ -757,10 +777,8 @@ void fwd_kernel(Fav4Args a, Layout L, int tiles, int total) {
         if constexpr (LSE) {
             if (half == 0 && row < a.sq) a.lse[int64_t(bh) * a.sq + row] = __builtin_fmaf(st.m, LN2, logf(st.l));
         }
-        wait_vmem();       // clamped prefetches and O stores have landed before the stages are reused
-        __syncthreads();
     };
-    for_each_item<CAUSAL>(tiles, total, process);
+    for_item<CAUSAL>(tiles, total, paired, process);
 }
 
 // ---------------------------------------------------------------------------
