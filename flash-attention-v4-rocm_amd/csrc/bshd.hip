@@ -119,13 +119,15 @@ constexpr int MAX_SPLIT_SQ = 1 << 22;    // keeps a chunk's O rows under a 4 GiB
 constexpr int DECODE_SQ = 32;            // up to this many queries: the one-wave decode shape
 
 // Tile shape of the partial kernel: 8 waves x 256-row q tiles x 64-key tiles
-// (one workgroup fills a CU), or for decode 1 wave x 32 rows x 32-key tiles
-// (three workgroups per CU, each with 48 KiB of LDS).
+// (one workgroup fills a CU), 4 waves x 128 rows (two per CU) where 256 rows
+// would leave half the waves without a query, or for decode 1 wave x 32 rows x
+// 32-key tiles (three workgroups per CU, each with 48 KiB of LDS).
 struct SplitShape {
     int bm, bn, wgs_per_cu, auto_max;
 };
 SplitShape split_shape(const Fav4Args& a) {
-    return a.sq <= DECODE_SQ ? SplitShape{32, 32, 3, 128} : SplitShape{256, 64, 1, 64};
+    if (a.sq <= DECODE_SQ) return {32, 32, 3, 128};
+    return {256, 64, 1, 64};
 }
 
 struct SplitPlan {
@@ -271,51 +273,66 @@ int split_args_ok(const Fav4Args* a, int kv_heads, int causal, int splits) {
     return st != hipSuccess ? st : split_shape_ok(a, kv_heads, causal, splits);
 }
 
+// Prefill chunks: K/V in BSHD (KV 0), packed (1) or paged (2) layout.
+template <bool CAUSAL, int KV, bool BR, int WAVES, int STAGES = 2>
+void launch_chunks(const Fav4Args& a, int kv_heads, const SplitPlan& p, const fav4::SplitArgs& sp, int64_t total,
+                   hipStream_t stream) {
+    const int tiles = (a.sq + WAVES * 32 - 1) / (WAVES * 32);
+    int key_bits = 1;
+    while (p.tps >> key_bits) ++key_bits;
+    if (a.lse)
+        hipLaunchKernelGGL((fav4::fwd_kernel_chunk<CAUSAL, true, WAVES, KV, BR, STAGES>), item_grid(total), dim3(WAVES * 64),
+                           0, stream, a, sp, kv_heads, tiles, int(total), key_bits);
+    else
+        hipLaunchKernelGGL((fav4::fwd_kernel_chunk<CAUSAL, false, WAVES, KV, BR, STAGES>), item_grid(total), dim3(WAVES * 64),
+                           0, stream, a, sp, kv_heads, tiles, int(total), key_bits);
+}
+
 // VARLEN: `a` holds the packed batch's shape (max lengths) and `sp` its
-// sequence offsets; decode shape only.  PAGED: the same over paged K/V caches.
+// sequence offsets.  PAGED: the same over paged K/V caches.
 // Top-left causal decode (sq <= 32) sees at most 32 keys, one tile, so the
-// plan never splits it: causal launches use the prefill shape only.
-// BR (packed decode only): bottom-right causal, the one causal mask a decode
-// splits.
+// plan never splits it: top-left causal launches use the prefill shape only.
+// BR (packed only): bottom-right causal.
 template <bool CAUSAL, bool VARLEN = false, bool PAGED = false, bool BR = false>
 int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, fav4::SplitArgs sp,
                  hipStream_t stream) {
     static_assert(!(CAUSAL && VARLEN) || BR, "top-left causal decode never splits");
-    static_assert(!BR || (CAUSAL && VARLEN), "bottom-right causal is for packed decode");
+    static_assert(!BR || (CAUSAL && VARLEN), "bottom-right causal is for packed calls");
     static_assert(!PAGED || VARLEN, "paged caches hold packed sequences");
-    const int tiles = p.tiles;
-    const int64_t total = p.items * tiles * p.splits;
-    const int64_t rows = int64_t(a.batch) * a.heads * a.sq;
     const bool decode = p.shape.bm == 32;
+    const int64_t rows = int64_t(a.batch) * a.heads * a.sq;
+    int64_t total = p.items * p.tiles * p.splits;
     if (total > INT_MAX || rows > INT_MAX || (VARLEN && !PAGED && !BR && !decode) || (CAUSAL && !BR && decode))
         return hipErrorInvalidValue;
     sp.o_part = static_cast<float*>(ws);
     sp.lse_part = sp.o_part + int64_t(p.splits) * rows * fav4::D;
     sp.splits = p.splits;
     sp.tps = p.tps;
-    const int grid = int(total < MAX_GRID ? total : MAX_GRID);
+    sp.bm = decode ? 0 : p.shape.bm;
+    sp.mask = BR ? 2 : CAUSAL;
     // The FP32 sums only feed an LSE output.
-    auto go = [&](auto kernel, int threads) {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, a, sp, kv_heads, tiles, int(total));
-    };
-    if constexpr (VARLEN) {
-        if (decode && a.lse) go(fav4::fwd_kernel_split<32, BR, 1, true, true, PAGED, BR>, 64);
-        else if (decode) go(fav4::fwd_kernel_split<32, BR, 1, false, true, PAGED, BR>, 64);
-        if constexpr (PAGED || BR) {  // prefill over paged caches or with the bottom-right mask: 8 waves
-            if (!decode && a.lse) go(fav4::fwd_kernel_split<64, BR, 8, true, true, PAGED, BR>, 512);
-            else if (!decode) go(fav4::fwd_kernel_split<64, BR, 8, false, true, PAGED, BR>, 512);
+    if (!decode) {
+        if constexpr (!VARLEN || PAGED || BR) {
+            constexpr int KV = PAGED ? 2 : VARLEN ? 1 : 0;
+            // The sorted lists hold only the q tiles that exist.
+            if (VARLEN && a.batch <= fav4::MAX_SORTED_SEQS)
+                total = std::min(total, a.heads * p.splits *
+                                            ((sp.total_q + int64_t(a.batch) * (p.shape.bm - 1)) / p.shape.bm));
+            if (p.shape.bm == 128) launch_chunks<CAUSAL, KV, BR, 4>(a, kv_heads, p, sp, total, stream);
+            else launch_chunks<CAUSAL, KV, BR, 8, KV == 0 ? 3 : 2>(a, kv_heads, p, sp, total, stream);
         }
-    } else if constexpr (CAUSAL) {
-        if (a.lse) go(fav4::fwd_kernel_split<64, true, 8, true>, 512);
-        else go(fav4::fwd_kernel_split<64, true, 8, false>, 512);
     } else {
-        if (decode && a.lse) go(fav4::fwd_kernel_split<32, false, 1, true>, 64);
-        else if (decode) go(fav4::fwd_kernel_split<32, false, 1, false>, 64);
-        else if (a.lse) go(fav4::fwd_kernel_split<64, false, 8, true>, 512);
-        else go(fav4::fwd_kernel_split<64, false, 8, false>, 512);
+        const int grid = int(total < MAX_GRID ? total : MAX_GRID), tiles = p.tiles;
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, a, sp, kv_heads, tiles, int(total));
+        };
+        if constexpr (!CAUSAL || BR) {
+            if (a.lse) go(fav4::fwd_kernel_split<32, BR, 1, true, VARLEN, PAGED, BR>);
+            else go(fav4::fwd_kernel_split<32, BR, 1, false, VARLEN, PAGED, BR>);
+        }
     }
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || (!decode && p.splits == 1)) return e;
     // Lane groups per merged row: one per 8 chunks, at most 8 (one workgroup).
     const int per = p.splits <= 8 ? 1 : p.splits <= 16 ? 2 : p.splits <= 32 ? 4 : 8;
     const int64_t row_blocks = (rows * per + 7) / 8;
@@ -430,6 +447,62 @@ SplitPlan packed_split_plan(const Fav4Args& a, int kv_heads, int64_t total_k, in
         p.splits = (ktiles + p.tps - 1) / p.tps;
     }
     return p;
+}
+
+// How the prefill of a packed or paged batch (max_seqlen_q > 32) with plan `p`
+// runs: the q tile (128 or 256 rows) and, for Auto, the chunk count up to the
+// plan's (which sizes the workspace) with the lowest predicted time.  The
+// plan takes every sequence as long as the longest; this model takes the
+// batch's means as well (microseconds, graph-timed on MI355X; a chunk costs
+// 9-10 plus c per key tile; a merged row's chunks are written and read once
+// more):
+//  * lengths near the longest (mean >= 3/4): whole rounds of equal chunks;
+//  * else the average load per resident workgroup plus a tenth of the longest
+//    item, or that item (the lists start the long items first).
+// On eight batches (1-8 sequences of 86-2048 queries against 1k-32k keys, H16
+// and H32) over 1-16 chunks and both tiles it picks the fastest measured choice
+// or one within 9% of it.  Merging costs what a second pass over FP32 partials
+// does: 4 x 1024 queries against 4096 keys H32 217 us in one chunk, 290 in two.
+SplitPlan packed_prefill_run(const Fav4Args& a, int64_t total_q, int64_t total_k, bool br, const SplitPlan& p,
+                             bool choose) {
+    const int ktiles = (a.sk + 63) / 64;
+    const double cus = device_cus(), seqs = a.batch;
+    const double mean_q = std::min<double>(a.sq, double(total_q) / seqs);
+    const double mean_k = std::min<double>(a.sk, double(total_k) / seqs);
+    const bool uniform = 4 * mean_k >= 3.0 * a.sk;
+    const double mean = std::max(1.0, mean_k / 64 + 0.5 - (br ? 0.5 * mean_q / 64 : 0.0));   // key tiles per q tile
+    auto predict = [&](int bm, int splits, int tps) {
+        const double slots = bm == 256 ? cus : 2 * cus;
+        const double qtiles = a.heads * std::min(seqs * ((a.sq + bm - 1) / bm), double(total_q) / bm + 0.5 * seqs);
+        const double chunks = std::max(1.0, std::ceil(mean / tps - 0.25)), items = qtiles * chunks;
+        const double fixed = bm == 256 ? 9.0 : 10.0;
+        const double per_tile = bm == 256 ? (a.sq > 128 ? 1.7 : 1.1) : (items > cus ? 1.75 : 1.1);
+        double t;
+        if (uniform) {
+            t = std::ceil(items / slots) * (fixed + per_tile * std::min<double>(tps, mean));
+        } else {
+            const double longest = fixed + std::min(per_tile, bm == 256 ? 1.6 : 1.4) * tps;
+            t = std::max(longest, qtiles * (chunks * fixed + per_tile * mean) / slots + 0.1 * longest);
+        }
+        if (splits > 1)
+            t += 5.0 + double(total_q) * a.heads * splits * 1040 / 4.5e6 *
+                           (uniform ? 1.0 : std::max(0.3, mean_k / a.sk));
+        return t;
+    };
+    SplitPlan best = p;
+    double best_t = 0;
+    bool first = true;
+    for (int s = choose ? 1 : p.splits; s <= p.splits; ++s) {
+        const int tps = s == p.splits ? p.tps : (ktiles + s - 1) / s, splits = (ktiles + tps - 1) / tps;
+        for (int bm : {256, 128}) {
+            const double t = predict(bm, splits, tps);
+            if (!first && t >= best_t) continue;
+            first = false;
+            best_t = t;
+            best = {splits, tps, SplitShape{bm, 64, bm == 256 ? 1 : 2, 64}, (a.sq + bm - 1) / bm, p.items};
+        }
+    }
+    return best;
 }
 
 // Bottom-right causal in the split-KV packed calls sees as many keys as a
@@ -718,6 +791,10 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
     sp.cu_k = a->cu_seqlens_k;
     sp.total_q = a->total_q;
     sp.total_k = a->total_k;
+    if (br && shape.sq > DECODE_SQ)
+        return launch_split<true, true, false, true>(
+            shape, a->kv_heads, packed_prefill_run(shape, a->total_q, a->total_k, true, p, splits == 0), workspace, sp,
+            stream);
     return br ? launch_split<true, true, false, true>(shape, a->kv_heads, p, workspace, sp, stream)
               : launch_split<false, true>(shape, a->kv_heads, p, workspace, sp, stream);
 }
@@ -742,7 +819,7 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
                                                                               hipStream_t stream) {
     const int st = paged_ok(a, causal, splits);
     if (st != hipSuccess) return st;
-    const SplitPlan p = paged_plan(*a, causal, splits);
+    SplitPlan p = paged_plan(*a, causal, splits);
     const int64_t need = paged_workspace(*a, p);
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255) || uint64_t(need) > workspace_bytes)
         return hipErrorInvalidValue;
@@ -754,9 +831,11 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
     sp.page_size = a->page_size;
     sp.max_pages = a->max_pages_per_seq;
     sp.num_pages = a->num_pages;
-    return causal == BOTTOM_RIGHT
-               ? launch_split<true, true, true, true>(paged_shape(*a), a->kv_heads, p, workspace, sp, stream)
-               : launch_split<false, true, true>(paged_shape(*a), a->kv_heads, p, workspace, sp, stream);
+    const Fav4Args shape = paged_shape(*a);
+    const bool br = causal == BOTTOM_RIGHT;
+    if (shape.sq > DECODE_SQ) p = packed_prefill_run(shape, a->total_q, a->total_k, br, p, splits == 0);
+    return br ? launch_split<true, true, true, true>(shape, a->kv_heads, p, workspace, sp, stream)
+              : launch_split<false, true, true>(shape, a->kv_heads, p, workspace, sp, stream);
 }
 
 // ---- Split-KV without a caller workspace ------------------------------------

@@ -164,6 +164,34 @@ __device__ __forceinline__ void packed_head_rank(int id, int heads, int& head, i
     }
 }
 
+// Items of a packed batch too large for the lists: `units` for every
+// (sequence, head), also those that its own lengths leave empty.  Each XCD
+// gets a contiguous run of them (a pair's units together, for its L2), but the
+// runs are cut from the pairs taken column by column from an 8-wide grid,
+// bh = 8*row + col: XCD x holds mostly the pairs with bh % 8 == x, i.e. a
+// share of every sequence rather than a few whole sequences, so ragged lengths
+// do not leave XCDs idle.
+__device__ __forceinline__ void column_item(int id, int total, int batch, int heads, int units, int& seq, int& head,
+                                            int& unit) {
+    const int nbh = batch * heads, full = nbh >> 3, rem8 = nbh & 7;
+    const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
+    const int logical = xcd * per + min(xcd, rem) + slot;
+    const int j = __builtin_amdgcn_readfirstlane(logical / units);
+    unit = __builtin_amdgcn_readfirstlane(logical - j * units);
+    int gcol, grow;
+    if (j < rem8 * (full + 1)) {
+        gcol = j / (full + 1);
+        grow = j - gcol * (full + 1);
+    } else {
+        const int jj = j - rem8 * (full + 1);
+        gcol = rem8 + jj / full;
+        grow = jj - (gcol - rem8) * full;
+    }
+    const int bh = grow * 8 + gcol;
+    seq = bh / heads;
+    head = bh - seq * heads;
+}
+
 // Byte strides of Q, K, V and O seen as [B, S, H, 128] (the 128 head dims
 // contiguous).  Row = one sequence position of one head.  BSHD: row stride
 // heads*256 (K/V: kv_heads*256), batch stride S*row, head stride 256.
@@ -523,6 +551,35 @@ __device__ __forceinline__ void store_o_rows(const RowState& st, float inv, unsi
     }
 }
 
+// The same for a key chunk's FP32 partial rows (512 bytes each, contiguous):
+// four rounds of 32 rows x 128 bytes, each store writing 8 rows x 128 bytes.
+// Straight from the accumulator an instruction wrote 32 rows x 32 bytes.
+template <int TILE_BYTES, bool LANE_OPAQUE>
+__device__ __forceinline__ void store_part_rows(const RowState& st, float inv, unsigned char* smem, uint32_t slot,
+                                                rsrc_t rp, int wrow0, int rows, int lane) {
+    static_assert(TILE_BYTES >= 16 * 128, "staging rows");
+    if constexpr (LANE_OPAQUE) asm volatile("" : "+v"(lane));
+    const int col = lane & 31, half = lane >> 5;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+#pragma unroll
+        for (int vg = 0; vg < 4; ++vg) {
+            const f32x4 x = {st.o[db][vg * 4 + 0] * inv, st.o[db][vg * 4 + 1] * inv,
+                             st.o[db][vg * 4 + 2] * inv, st.o[db][vg * 4 + 3] * inv};
+            const uint32_t off = slot + (col >> 4) * TILE_BYTES + (col & 15) * 128 +
+                                 (((2 * vg + half) ^ (col & 7)) << 4);
+            *reinterpret_cast<FAV4_LDS f32x4*>((FAV4_LDS void*)(smem + off)) = x;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 8 * i + (lane >> 3), c = lane & 7;
+            const uint32_t off = slot + (r >> 4) * TILE_BYTES + (r & 15) * 128 + ((c ^ (r & 7)) << 4);
+            const f32x4 v = *reinterpret_cast<const FAV4_LDS f32x4*>((FAV4_LDS const void*)(smem + off));
+            if (r < rows) store16(rp, uint32_t(wrow0 + r) * (D * 4) + db * 128 + c * 16, v);
+        }
+    }
+}
+
 // WAVES waves x 32 query rows per workgroup, BN keys per tile, STAGES LDS
 // buffers of K+V.  Tile t lives in stage t % STAGES; its DMA is issued
 // STAGES-1 tiles ahead (right after barrier t-STAGES+1, into the stage that
@@ -814,19 +871,23 @@ struct SplitArgs {
     const int* seqlens_k;
     const int* block_table;
     int page_size, max_pages, num_pages;
+    // What the merge needs to count a prefill row's chunks: query rows per q
+    // tile (0: decode, every chunk is merged) and the mask (0 dense, 1
+    // top-left, 2 bottom-right).
+    int bm, mask;
 };
 
 // Query / key count and first token of sequence b (the same in every lane of
-// the workgroup), read on the device and clamped to [0, total] and to the max
+// the workgroup unless PER_LANE), read on the device and clamped to [0, total] and to the max
 // lengths, as fwd_kernel_varlen does.  PAGED: the key count is seqlens_k[b]
 // clamped to [0, max_k] (ktok unused).
 struct SeqSpan {
     int sq, sk;
     int64_t qtok, ktok;
 };
-template <bool PAGED>
+template <bool PAGED, bool PER_LANE = false>
 __device__ __forceinline__ SeqSpan seq_span(const SplitArgs& sp, int b, int max_q, int max_k) {
-    auto rd = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    auto rd = [](int x) { return PER_LANE ? x : __builtin_amdgcn_readfirstlane(x); };
     const int qs = min(max(rd(sp.cu_q[b]), 0), sp.total_q);
     const int qe = min(max(rd(sp.cu_q[b + 1]), qs), min(sp.total_q, qs + max_q));
     if constexpr (PAGED) return {qe - qs, min(max(rd(sp.seqlens_k[b]), 0), max_k), qs, 0};
@@ -1078,6 +1139,235 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
 
 #pragma clang diagnostic pop
 
+// Keys that the queries [q0, q0 + bm) of a sequence can see (mask 0 dense, 1
+// top-left causal, 2 bottom-right causal).  Never more than its last query
+// sees, which is what the plan's chunks cover.
+__device__ __forceinline__ int visible_keys(int mask, int q0, int bm, int sq, int sk) {
+    if (mask == 0) return sk;
+    if (mask == 1) return min(sk, min(sq, q0 + bm));
+    return min(sk, max(0, min(sq, q0 + bm) + sk - sq));
+}
+
+// Prefill chunks (more than 32 queries): WAVES x 32 query rows of one head
+// against one chunk of sp.tps 64-key tiles.  A q tile whose visible keys fit
+// one chunk writes its O and LSE itself, bitwise what the merge of that one
+// chunk gives; the others write their partials row-contiguously for
+// combine_kernel.
+// STAGES: BSHD calls, whose few q tiles mostly stream K/V, keep three LDS
+// stages (prefetch distance 2; B2 H16 128 x 65536 200 us, 212 with two); packed
+// and paged ones, which fill the GPU, run two (4 x 1024 x 4096 H32 205 us, 211
+// with three).
+// KV: where K/V lie.  0: BSHD, 1: packed sequences, 2: paged caches.  Packed
+// and paged items come from the sequences' lengths (sorted_item), heaviest
+// chunks first, so that a sequence with few keys or queries costs what it has:
+// against a grid up to the longest lengths, three stages and a merge of every
+// row, 4 chunks of 517..1024 queries on 1.3k-8.2k keys H32/8 253 -> 183 us,
+// 8 x 128 queries on 1k-16k keys 250 -> 133.
+// BR (with KV > 0): bottom-right causal.
+// Paged: page_size is a multiple of 64, so a key tile lies in one page; one
+// load puts the (clamped) numbers of 64 pages in the wave's lanes.
+template <bool CAUSAL, bool LSE, int WAVES, int KV, bool BR, int STAGES = 2>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void fwd_kernel_chunk(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int total, int key_bits) {
+    static_assert(!BR || (CAUSAL && KV), "bottom-right causal needs per-sequence lengths");
+    constexpr int BN = 64, BM = WAVES * 32, MASK = BR ? 2 : CAUSAL;
+    constexpr int TILE_BYTES = BN * ROW_BYTES;
+    constexpr int STAGE_BYTES = 2 * TILE_BYTES;
+    constexpr int DMA = BN / 4 / WAVES;
+    static_assert(DMA >= 2, "a wave's DMA slots hold 2 KiB per matrix (O staging)");
+    static_assert(STAGES == 2 || STAGES == 3, "stages");
+    constexpr int AHEAD = STAGES - 1;                      // prefetch distance in tiles
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[STAGES * STAGE_BYTES];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 31, half = lane >> 5;
+    const uint32_t row_bytes = uint32_t(a.heads) * ROW_BYTES;
+    const uint32_t kv_row_bytes = uint32_t(kv_heads) * ROW_BYTES;
+    const int group = a.heads / kv_heads;
+    const float scale2 = a.scale * LOG2E;
+    const uint32_t smem_base = lds_addr(smem);
+    const int bhs = a.batch * a.heads;
+
+    // The item: (sequence, head, q tile, chunk), one per workgroup.
+    const int id = int(blockIdx.y * gridDim.x + blockIdx.x);
+    if (id >= total) return;
+    int batch, head, unit, ntile = tiles;
+    SeqSpan span;
+    if constexpr (KV == 0) {
+        // XCD-contiguous order; the q tiles of one (b, h) chunk are adjacent,
+        // so they share it in L2.
+        const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
+        const int logical = xcd * per + min(xcd, rem) + slot;
+        const int per_item = tiles * sp.splits;
+        const int it = logical / per_item;
+        unit = logical - it * per_item;
+        batch = it / a.heads;
+        head = it - batch * a.heads;
+        span = {a.sq, a.sk, int64_t(batch) * a.sq, int64_t(batch) * a.sk};
+    } else if (a.batch <= MAX_SORTED_SEQS) {
+        int rank;
+        packed_head_rank(id, a.heads, head, rank);
+        const PackedItem it = sorted_item<BM, BN>(rank, a.batch, key_bits, lane, [&](int b) {
+            const SeqSpan s = seq_span<KV == 2, true>(sp, b, a.sq, a.sk);
+            const int nt = (s.sq + BM - 1) / BM, nk = (s.sk + BN - 1) / BN;
+            const int chunks = max(1, (nk + sp.tps - 1) / sp.tps);
+            return PackedSeq{Span{int(s.qtok), int(s.qtok) + s.sq, int(s.ktok), int(s.ktok) + s.sk}, nt * chunks,
+                             min(s.sk, sp.tps * BN), INT_MAX};
+        });
+        if (it.seq < 0) return;
+        batch = it.seq;
+        unit = it.place;
+        span = {it.span.qe - it.span.qs, it.span.ke - it.span.ks, it.span.qs, it.span.ks};
+        ntile = (span.sq + BM - 1) / BM;
+    } else {
+        column_item(id, total, a.batch, a.heads, tiles * sp.splits, batch, head, unit);
+        span = seq_span<KV == 2>(sp, batch, a.sq, a.sk);
+    }
+    auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    batch = uniform(batch), head = uniform(head), unit = uniform(unit);
+    const int split = uniform(unit / ntile), place = unit - split * ntile;
+    const int tile = KV == 0 ? place : ntile - 1 - place;     // packed: heaviest first
+    const int sq = uniform(span.sq), sk = uniform(span.sk);
+    const int q0 = tile * BM, qw = q0 + wave * 32;
+    if (q0 >= sq) return;
+    const int row = qw + col;
+    const int shift = BR ? sk - sq : 0;
+    const int kend = visible_keys(MASK, q0, BM, sq, sk);
+    const int ntiles = (kend + BN - 1) / BN;
+    const int t0 = split * sp.tps, t1 = min(ntiles, t0 + sp.tps);
+    const bool direct = ntiles <= sp.tps;
+    if (t0 >= t1 && split > 0) return;                     // past what this q tile sees
+    // Tiles below nfull are unmasked for every row of the q tile.
+    const int nfull = (MASK == 0 ? sk : max(0, min(sk, q0 + 1 + shift))) / BN;
+    const int climit = row + shift;                        // last visible key of this lane's row (causal)
+
+    const int64_t qtok = KV == 0 ? int64_t(batch) * a.sq : int64_t(uniform(int(span.qtok)));
+    const int64_t ktok = KV == 0 ? int64_t(batch) * a.sk : int64_t(uniform(int(span.ktok)));
+    const int64_t qrow0 = (qtok + q0) * a.heads + head;
+    const int64_t krow0 = ktok * kv_heads + head / group;
+    const char* kbase = static_cast<const char*>(a.k) + krow0 * ROW_BYTES;
+    const char* vbase = static_cast<const char*>(a.v) + krow0 * ROW_BYTES;
+    const uint32_t qbytes = uint32_t(sq - q0 - 1) * row_bytes + ROW_BYTES;
+
+    const LdsOffsets off = lds_offsets(lane);
+    const DmaOffsets<DMA> dofs = dma_offsets<DMA>(wave, lane, kv_row_bytes, kv_row_bytes);
+    RowState st;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) st.o[db] = f32x16{};
+    st.m = -__builtin_inff();
+    st.lb = 0.f;
+    st.l = 0.f;
+
+    if (t0 < t1) {
+        // Paged: lane l holds the page of slot page0 + l, for 64 slots at a time.
+        int pages = 0, page0 = 0;
+        auto load_pages = [&](int slot0) {
+            page0 = slot0;
+            const int slot = min(page0 + lane, sp.max_pages - 1);
+            pages = min(max(sp.block_table[int64_t(batch) * sp.max_pages + slot], 0), sp.num_pages - 1);
+        };
+        if constexpr (KV == 2) load_pages(t0 * BN / sp.page_size);
+        // Three stages: tiles past the chunk are clamped to its last one (the
+        // copy lands in a stage no later step reads), which keeps the vmcnt
+        // count uniform.
+        auto issue = [&](int t) {
+            const uint32_t stage = smem_base + ((t - t0) % STAGES) * STAGE_BYTES;
+            if constexpr (STAGES > 2) t = min(t, t1 - 1);
+            int64_t row0 = int64_t(t) * BN;                 // the tile's first K/V row
+            int rows_left = sk - t * BN;                    // rows the descriptor may cover
+            if constexpr (KV == 2) {
+                const int first = t * BN, slot = first / sp.page_size, in_page = first - slot * sp.page_size;
+                if (slot - page0 >= 64) load_pages(slot);
+                row0 = int64_t(__builtin_amdgcn_readlane(pages, slot - page0)) * sp.page_size + in_page;
+                rows_left = min(rows_left, sp.page_size - in_page);
+            }
+            const uint32_t bytes = uint32_t(rows_left - 1) * kv_row_bytes + ROW_BYTES;
+            const u32x4 rk = make_desc(kbase + row0 * kv_row_bytes, bytes);
+            const u32x4 rv = make_desc(vbase + row0 * kv_row_bytes, bytes);
+            dma_tile<DMA, TILE_BYTES>(rk, rv, stage, wave, dofs);
+        };
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) issue(t0 + i);
+        bf16x8 qr[8];
+        {
+            const rsrc_t rq = make_rsrc(static_cast<const char*>(a.q) + qrow0 * ROW_BYTES, qbytes);
+            const uint32_t qoff = uint32_t(wave * 32 + col) * row_bytes + half * 16;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) qr[c] = load16(rq, qoff + c * 32);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) asm volatile("" ::"v"(qr[c]));
+        }
+        auto sync_and_prefetch = [&](int t) {
+            wait_vmem_keep<2 * DMA * (AHEAD - 1)>();
+            __syncthreads();
+            if (STAGES > 2 || t + 1 < t1) issue(t + AHEAD);
+        };
+        auto step = [&](auto stage_c, auto masked_c, int t) {
+            constexpr int STAGE = decltype(stage_c)::value;
+            const unsigned char* cur = smem + STAGE * STAGE_BYTES;
+            sync_and_prefetch(t);
+            // A causal tile entirely above this wave's rows changes nothing.
+            if (!(decltype(masked_c)::value && CAUSAL) || t * BN <= qw + 31 + shift)
+                attend_fused<BN, decltype(masked_c)::value, CAUSAL, LSE, CAUSAL>(
+                    cur, cur + TILE_BYTES, off, qr, st, t == t0, t * BN, sk, climit, half, scale2);
+        };
+        using S0 = std::integral_constant<int, 0>;
+        using S1 = std::integral_constant<int, 1>;
+        using S2 = std::integral_constant<int, 2 % STAGES>;
+        using Plain = std::integral_constant<bool, false>;
+        using Masked = std::integral_constant<bool, true>;
+        int t = t0;
+        const int tp = min(t1, nfull);
+        if (qw >= sq) {
+            // Rows all past the queries: only the DMA and barrier sequence.
+            for (; t < t1; ++t) sync_and_prefetch(t);
+        } else {
+            // Steps in compile-time stage groups, the masked ones too
+            // ((t - t0) % STAGES is 0 there), so O keeps one register home.
+            auto group = [&](auto masked, int end) {
+                for (; t + AHEAD < end; t += STAGES) {
+                    step(S0{}, masked, t);
+                    step(S1{}, masked, t + 1);
+                    if constexpr (STAGES == 3) step(S2{}, masked, t + 2);
+                }
+            };
+            group(Plain{}, tp);
+            group(Masked{}, t1);
+            if (t < t1) step(S0{}, Masked{}, t);
+            if constexpr (STAGES == 3)
+                if (t + 1 < t1) step(S1{}, Masked{}, t + 1);
+        }
+    }
+
+    // The last tile of stage (t1 - t0) % STAGES was read before the last step's
+    // barrier and it receives at most a clamped prefetch: once this wave's own
+    // part of that has landed, its slots there hold the staging.
+    if constexpr (STAGES > 2) wait_vmem();
+    const float inv = st.lb > 0.f ? 1.f / st.lb : 0.f;
+    const uint32_t slot = uint32_t((max(0, t1 - t0) % STAGES) * STAGE_BYTES + wave * DMA * 1024);
+    const bool mine = half == 0 && row < sq;
+    if (direct) {
+        const rsrc_t ro = make_rsrc(static_cast<char*>(a.o) + qrow0 * ROW_BYTES, qbytes);
+        store_o_rows<TILE_BYTES, LSE>(st, inv, smem, slot, ro, row_bytes, wave * 32, sq - qw, lane);
+        if constexpr (LSE) {
+            const int64_t at = KV == 0 ? (int64_t(batch) * a.heads + head) * a.sq + row
+                                       : int64_t(head) * sp.total_q + qtok + row;
+            if (mine) a.lse[at] = (st.m + __builtin_amdgcn_logf(st.l)) * LN2;
+        }
+    } else {
+        const int64_t prow0 = (int64_t(split) * bhs + int64_t(batch) * a.heads + head) * a.sq + q0;
+        const rsrc_t rp = make_rsrc(sp.o_part + prow0 * D, uint32_t(sq - q0) * D * 4);
+        store_part_rows<TILE_BYTES, LSE>(st, inv, smem, slot, rp, wave * 32, sq - qw, lane);
+        if (mine) {
+            float* lp = sp.lse_part + (prow0 + row - q0) * 2;
+            const float sb = st.m + __builtin_amdgcn_logf(st.lb);
+            lp[0] = sb;
+            lp[1] = LSE ? st.m + __builtin_amdgcn_logf(st.l) : sb;
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Varlen: packed sequences.  Q/O are [total_q, heads, 128] and K/V
 // [total_k, kv_heads, 128]; sequence b owns rows [cu_seqlens_q[b],
@@ -1126,7 +1416,12 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
     // tile weighs its key tiles (by_item: with few items per workgroup slot,
     // where the last ones decide) or its sequence's longest tile's (its q
     // tiles then run together, heaviest first, and share its K/V in L2).
-    // Against the order below (graph-timed, causal): 24 sequences of 64..4096
+    // Against that order (graph-timed, causal): 24 sequences of 64..4096
+    // tokens H32 KVH8 708 -> 582 us, 64 of 100..1000 H8 69 -> 55, 4 x 2048
+    // H16 105 -> 77 (by sequence 97), 8 x 4096 H8 313 -> 264 (313); 32 of
+    // 1024..7168 H8 858 -> 848.
+    // Larger batches: column_item.
+    // Against that order (graph-timed, causal): 24 sequences of 64..4096
     // tokens H32 KVH8 708 -> 582 us, 64 of 100..1000 H8 69 -> 55, 4 x 2048
     // H16 105 -> 77 (by sequence 97), 8 x 4096 H8 313 -> 264 (313); 32 of
     // 1024..7168 H8 858 -> 848.
@@ -1138,10 +1433,7 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
     // ragged lengths do not leave XCDs idle.  Within a pair the q tiles run
     // last-to-first (causal: heaviest first).
     const bool sorted = a.batch <= MAX_SORTED_SEQS;
-    const int nbh = a.batch * a.heads, full = nbh >> 3, rem8 = nbh & 7;
     {
-        // One item per workgroup (no loop over items: the state it would keep
-        // live through the key loop costs that loop its V reads' depth).
         const int id = int(blockIdx.y * gridDim.x + blockIdx.x);
         if (id >= total) return;
         int batch, head, tile;
@@ -1161,22 +1453,9 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
             sp = it.span;
             tile = (sp.qe - sp.qs + BM - 1) / BM - 1 - it.place;       // from the last q tile down
         } else {
-            const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
-            const int logical = xcd * per + min(xcd, rem) + slot;
-            const int j = __builtin_amdgcn_readfirstlane(logical / tiles);
-            tile = __builtin_amdgcn_readfirstlane(tiles - 1 - (logical - j * tiles));
-            int gcol, grow;
-            if (j < rem8 * (full + 1)) {
-                gcol = j / (full + 1);
-                grow = j - gcol * (full + 1);
-            } else {
-                const int jj = j - rem8 * (full + 1);
-                gcol = rem8 + jj / full;
-                grow = jj - (gcol - rem8) * full;
-            }
-            const int bh = grow * 8 + gcol;
-            batch = bh / a.heads;
-            head = bh - batch * a.heads;
+            int unit;
+            column_item(id, total, a.batch, a.heads, tiles, batch, head, unit);
+            tile = tiles - 1 - unit;
             sp = span(batch);
         }
         batch = __builtin_amdgcn_readfirstlane(batch);
@@ -1333,14 +1612,25 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
         const int batch = int(bh / a.heads), head = int(bh - int64_t(batch) * a.heads);
         int64_t qtok = int64_t(batch) * a.sq + qi;       // the row's token (BSHD)
         bool live = r < rows;
+        int sq = a.sq, sk = a.sk, nch = sp.splits;
         if constexpr (VARLEN) {
             if (live) {
-                // Only the query side: paged batches have no key offsets.
+                // Only prefill needs the key count; paged batches have no key offsets.
                 const int qs = min(max(sp.cu_q[batch], 0), sp.total_q);
-                const int qe = min(max(sp.cu_q[batch + 1], qs), min(sp.total_q, qs + a.sq));
-                live = qi < qe - qs;
+                sq = min(max(sp.cu_q[batch + 1], qs), min(sp.total_q, qs + a.sq)) - qs;
+                if (sp.bm) sk = (sp.seqlens_k ? seq_span<true, true>(sp, batch, a.sq, a.sk)
+                                              : seq_span<false, true>(sp, batch, a.sq, a.sk)).sk;
+                live = qi < sq;
                 qtok = int64_t(qs) + qi;
             }
+        }
+        if (sp.bm && (VARLEN || sp.mask)) {
+            // A q tile of one chunk was written by it; the others have as many
+            // chunks as their visible keys (BSHD dense: all have sp.splits).
+            const int vis = visible_keys(sp.mask, qi - qi % sp.bm, sp.bm, sq, sk);
+            nch = min(sp.splits, ((vis + 63) / 64 + sp.tps - 1) / sp.tps);
+            if (nch <= 1) live = false;
+            if (!__syncthreads_or(live)) continue;
         }
         // The partial O rows do not depend on the weights: their loads go out
         // first, so that their latency overlaps the log-sum phase (one memory
@@ -1351,7 +1641,7 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
             const int s = part + i * PER;
-            xo[i] = live && s < sp.splits ? *reinterpret_cast<const f32x4*>(op + s * slab * D) : f32x4{};
+            xo[i] = live && s < nch ? *reinterpret_cast<const f32x4*>(op + s * slab * D) : f32x4{};
         }
         float vb[MAXV], vl[MAXV];
         float mb = -__builtin_inff(), ml = -__builtin_inff();
@@ -1359,7 +1649,7 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
         for (int i = 0; i < MAXV; ++i) {
             const int s = team + i * NT;
             vb[i] = vl[i] = -__builtin_inff();
-            if (live && s < sp.splits) {
+            if (live && s < nch) {
                 const float2 v = *reinterpret_cast<const float2*>(sp.lse_part + (s * slab + r) * 2);
                 vb[i] = v.x;
                 vl[i] = v.y;
@@ -1384,7 +1674,7 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
 #pragma unroll
         for (int i = 0; i < MAXV; ++i) {
             const int s = team + i * NT;
-            if (s < sp.splits) {
+            if (s < nch) {
                 const float w = live ? exp2_native(vb[i] - mb) : 0.f;
                 wsh[slot][s] = w;
                 den += w;
@@ -1409,7 +1699,7 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
 #pragma unroll
             for (int i = 0; i < NS; ++i) {
                 const int s = part + i * PER;
-                if (s < sp.splits) {
+                if (s < nch) {
                     const float w = wsh[slot][s];
                     if (w > 0.f) acc += w * xo[i];
                 }

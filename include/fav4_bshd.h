@@ -177,10 +177,12 @@ extern "C" int fav4_bshd_forward_varlen(const Fav4VarlenArgs* args, int causal, 
 // query i of a sequence with sq queries and sk keys sees keys j <= sk - sq + i
 // (the last query sees them all; with sq > sk the first sq - sk rows see
 // none: O = 0, LSE = -inf).  Decode (max_seqlen_q <= 32) is planned like a
-// dense call; prefill (max_seqlen_q > 32, 8-wave kernels) with the contiguous
-// prefill plan at the max lengths, counting for each 256-row q tile only the
-// keys up to its last row's diagonal (chunks past it are empty and end at
-// once).  Decode always runs the split kernels, one chunk included (with a
+// dense call; prefill (max_seqlen_q > 32) with the contiguous prefill plan at
+// the max lengths, counting for each 256-row q tile only the keys up to its
+// last row's diagonal.  A prefill q tile whose visible keys fit one chunk is
+// written without a merge, and Auto may run fewer chunks than the plan that
+// sizes the workspace where the batch's mean lengths make that faster.
+// Decode always runs the split kernels, one chunk included (with a
 // workspace); prefill with one chunk runs fav4_bshd_forward_varlen, which
 // takes the same mask, and needs none.  Same argument contract
 // as fav4_bshd_forward_varlen (O and LSE rows, empty sequences, offset
@@ -213,9 +215,11 @@ extern "C" int fav4_bshd_splitkv_varlen_select(const Fav4VarlenArgs* args, int c
 // 32-row tiles; chunks of a common number of key tiles, merged by
 // log-sum-exp), so per row the result is bitwise that of
 // fav4_bshd_forward_splitkv_varlen on the same keys stored contiguously, at
-// the same chunk count.  Prefill runs the 8-wave split-KV kernels (256-row q
-// tiles, 64-key tiles) with the contiguous prefill plan at the max lengths,
-// bitwise fav4_bshd_forward_splitkv_gqa's on a batch of equal lengths.
+// the same chunk count.  Prefill runs the split-KV prefill kernels (128- or
+// 256-row q tiles, 64-key tiles) with the contiguous prefill plan at the max
+// lengths (Auto: that many chunks or fewer, as above), bitwise
+// fav4_bshd_forward_splitkv_gqa's on a batch of equal lengths at the same
+// explicit chunk count.
 struct Fav4PagedArgs {
     const void *q;                     // BF16 [total_q, heads, 128], contiguous
     const void *k_cache, *v_cache;     // BF16 [num_pages, page_size, kv_heads, 128], contiguous
@@ -234,7 +238,7 @@ struct Fav4PagedArgs {
 // sizes >= 1 (total_k >= 0), kv_heads dividing heads, causal 0 or 2, a finite
 // positive scale, max_seqlen_q <= 2^22, page_size a multiple of 32 (decode)
 // or 64 (prefill), max_seqlen_k <= max_pages_per_seq * page_size and <= 2^19
-// (a chunk spans at most 64 key tiles), page_size * kv_heads * 256 < 2^32,
+// (a plan's chunk spans at most 64 key tiles), page_size * kv_heads * 256 < 2^32,
 // max_seqlen_q * heads * 256 < 2^32, for decode (heads / kv_heads) *
 // max_seqlen_q < 2^23, 16-byte aligned Q/O/caches and 4-byte aligned int
 // arrays and LSE.
@@ -243,8 +247,8 @@ struct Fav4PagedArgs {
 // undefined results but no access outside the buffers.  A sequence with no
 // keys gets O = 0 and LSE = -inf; one with no queries writes nothing.
 //  * splits: 0 = the Auto count of fav4_bshd_forward_splitkv_varlen on these
-//    sizes, else 1..256; either is raised if needed so that no chunk spans
-//    more than 64 key tiles.  One chunk still runs the split kernels.
+//    sizes, else 1..256; either is raised if needed so that no chunk of the plan
+//    spans more than 64 key tiles.  One chunk still runs the split kernels.
 //  * workspace as for fav4_bshd_forward_splitkv, of
 //    fav4_bshd_splitkv_paged_workspace_size() bytes (never 0).
 // The two queries read only the sizes (pointers may be NULL) and return -1

@@ -376,3 +376,59 @@ def test_splitkv_paged_presized_workspace_bottom_right(gpu_runner):
     torch.cuda.synchronize()
     assert torch.equal(o.view(torch.int16), o2.view(torch.int16))
     assert torch.equal(lse.view(torch.int32), lse2.view(torch.int32))
+
+
+# (heads, kv_heads, page_size, [(sq, sk), ...]): q tiles that end in one chunk
+# beside q tiles that are merged, sizes at the edges of the 64-key and 128- /
+# 256-row tiles, queries without a visible key, few sequences (sorted item
+# lists) and more than 256 (plain grid), and a grid that Auto fills with one
+# chunk of more than 64 pages per q tile.
+PREFILL_CASES = [
+    (4, 2, 64, [(200, 9001), (129, 64), (33, 65), (255, 4097)]),
+    (8, 8, 64, [(257, 700), (256, 256), (128, 128), (1, 6000), (0, 500), (130, 0), (300, 90)]),
+    (8, 2, 128, [(1 + 37 * i % 70, 1 + 61 * i % 400) for i in range(260)]),
+    (32, 2, 64, [(256, 4500 + i) for i in range(8)]),
+]
+
+
+@pytest.mark.parametrize("case", PREFILL_CASES, ids=lambda c: "h%dkv%d_p%d_n%d" % (c[0], c[1], c[2], len(c[3])))
+def test_paged_prefill_chunks(gpu_runner, case):
+    """Bottom-right prefill over paged caches: in one chunk O is bitwise the
+    unsplit packed forward's (a q tile of one chunk writes its own O); with
+    more chunks it is within the reference bar (0.01 + 0.01 |ref|) of it, and
+    bitwise the packed K/V call's where the plans agree; nothing is written
+    past O and LSE."""
+    import torch
+    h, kvh, ps, lens = case
+    q, k, v, kc, vc, cu_q, cu_k, seqlens_k, table = _build(h, kvh, ps, lens, seed=97)
+    dev = torch.device("cuda:0")
+    qd, kd, vd, kcd, vcd = (to_device(x, dev) for x in (q, k, v, kc, vc))
+    cq, ck, sk_d, tb = (torch.from_numpy(x).to(dev) for x in (cu_q, cu_k, seqlens_k, table))
+    max_q, max_k, tq = max(s for s, _ in lens), max(s for _, s in lens), len(q)
+    whole_buf, _, whole, whole_lse = _out(torch, dev, tq, h, True)
+    gpu_runner.call_varlen(qd, kd, vd, whole, whole_lse, cq, ck, max_q, max_k, 2)
+    for splits in (1, 2, 5, 0):
+        print(f"  paged prefill h{h} kv{kvh} n{len(lens)} splits {splits}", flush=True)
+        ob, lb, o, lse = _out(torch, dev, tq, h, True)
+        gpu_runner.call_splitkv_paged(qd, kcd, vcd, o, lse, cq, sk_d, tb, max_q, max_k, splits, total_k=len(k),
+                                      causal=2)
+        ob2, _, o2, _ = _out(torch, dev, tq, h, False)
+        gpu_runner.call_splitkv_paged(qd, kcd, vcd, o2, None, cq, sk_d, tb, max_q, max_k, splits, total_k=len(k),
+                                      causal=2)
+        ob3, lb3, o3, lse3 = _out(torch, dev, tq, h, True)
+        gpu_runner.call_splitkv_varlen(qd, kd, vd, o3, lse3, cq, ck, max_q, max_k, 2, splits)
+        torch.cuda.synchronize()
+        for guard in (ob[tq:], ob2[tq:], ob3[tq:], lb[h * tq:], lb3[h * tq:]):
+            assert torch.isnan(guard).all().item(), splits
+        assert torch.equal(o.view(torch.int16), o2.view(torch.int16)), splits
+        sizes = (len(lens), h, kvh, max_q, max_k, tq, len(k))
+        ws_p = gpu_runner.splitkv_paged_workspace_size(*sizes, ps, table.shape[1], len(kc), splits, causal=2)
+        if ws_p == gpu_runner.splitkv_varlen_workspace_size(*sizes, 2, splits):
+            assert torch.equal(o.view(torch.int16), o3.view(torch.int16)), splits
+        if ws_p == len(lens) * h * max_q * 520:               # one chunk
+            assert torch.equal(o.view(torch.int16), whole.view(torch.int16))
+        else:
+            assert ((o.float() - whole.float()).abs() <= 0.01 + 0.01 * whole.float().abs()).all().item(), splits
+        seen = torch.isfinite(whole_lse)
+        assert torch.equal(torch.isfinite(lse), seen) and torch.equal(torch.isfinite(lse3), seen)
+        assert (lse[seen] - whole_lse[seen]).abs().max().item() <= 2e-4, splits
