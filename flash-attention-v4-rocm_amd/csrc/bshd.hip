@@ -135,6 +135,7 @@ struct SplitPlan {
     SplitShape shape;
     int tiles;         // q tiles per item
     int64_t items;     // (batch, head) items, or (batch, K/V head) groups for decode
+    int ranges = 0;    // decode over equal ranges of the packed keys: workgroups per (K/V head, q tile); 0: not
 };
 
 // Auto for prefill (Sq > 32).  Filling the CUs is not enough: on the small
@@ -321,6 +322,18 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
             if (p.shape.bm == 128) launch_chunks<CAUSAL, KV, BR, 4>(a, kv_heads, p, sp, total, stream);
             else launch_chunks<CAUSAL, KV, BR, 8, KV == 0 ? 3 : 2>(a, kv_heads, p, sp, total, stream);
         }
+    } else if (VARLEN && p.ranges > 0) {
+        if constexpr (VARLEN) {
+            const int ktiles = (a.sk + p.shape.bn - 1) / p.shape.bn;
+            const int min_tiles = (ktiles + p.splits - 2) / (p.splits - 1);
+            const dim3 grid(unsigned(kv_heads) * unsigned(p.tiles) * unsigned(p.ranges));
+            if (a.lse)
+                hipLaunchKernelGGL((fav4::fwd_kernel_ranges<true, PAGED, BR>), grid, dim3(64), 0, stream, a, sp,
+                                   kv_heads, p.tiles, p.ranges, min_tiles);
+            else
+                hipLaunchKernelGGL((fav4::fwd_kernel_ranges<false, PAGED, BR>), grid, dim3(64), 0, stream, a, sp,
+                                   kv_heads, p.tiles, p.ranges, min_tiles);
+        }
     } else {
         const int grid = int(total < MAX_GRID ? total : MAX_GRID), tiles = p.tiles;
         auto go = [&](auto kernel) {
@@ -447,6 +460,39 @@ SplitPlan packed_split_plan(const Fav4Args& a, int kv_heads, int64_t total_k, in
         p.splits = (ktiles + p.tps - 1) / p.tps;
     }
     return p;
+}
+
+// How Auto runs the decode of a packed or paged batch whose plan is `p` (which
+// sizes the workspace): equal ranges of the batch's keys, RANGE_WGS_PER_CU
+// one-wave workgroups per CU (fwd_kernel_ranges), unless
+//  * every sequence has the longest one's keys (the contiguous plan cuts those
+//    evenly, and its result is kept bitwise);
+//  * a range would be under MIN_RANGE_TILES key tiles: the short ranges' fixed
+//    cost then outweighs their balance (H32 KVH8, plan / ranges: 8.5 tiles, 32
+//    sequences of 64..2048 keys 28.5 / 26.2 us; 4.1 tiles, 3 of 2500..3000
+//    15.6 / 17.3; 2.5 tiles, 8 of 100..2000 15.0 / 16.4);
+//  * the plan's chunks would not hold the ranges: a sequence of n tiles meets
+//    at most (n - 2) / (range length) + 2 of them, so `splits` chunks suffice
+//    for ranges of at least ktiles / (splits - 1) tiles, which the kernel keeps
+//    to;
+//  * the batch has more sequences than a wave's lanes list.
+// Two workgroups per CU against three (the plan's): 32 sequences of 1k..32k
+// keys 207 and 210 us, 64 of 64..2048 38 and 41, 200 of 300..9000 337 and 341,
+// 16 of 8 queries H64 on 1k..16k 102 and 115; 8 of 1k..32k 87 and 86.
+constexpr int RANGE_WGS_PER_CU = 2;
+constexpr int MIN_RANGE_TILES = 8;
+SplitPlan packed_decode_run(const Fav4Args& a, int kv_heads, int64_t total_k, const SplitPlan& p) {
+    if (a.batch > fav4::MAX_SORTED_SEQS || p.splits < 2 || total_k >= int64_t(a.batch) * a.sk) return p;
+    const int64_t streams = int64_t(kv_heads) * p.tiles;
+    const int64_t ranges = int64_t(device_cus()) * RANGE_WGS_PER_CU / streams;
+    if (ranges < 2) return p;
+    const int64_t ktiles = (a.sk + p.shape.bn - 1) / p.shape.bn;
+    const int64_t range = (total_k / p.shape.bn + a.batch / 2 + ranges - 1) / ranges;
+    if (range < MIN_RANGE_TILES || ktiles > range * (p.splits - 1)) return p;
+    SplitPlan run = p;
+    run.splits = int(std::min<int64_t>(p.splits, (ktiles + range - 1) / range + 2));
+    run.ranges = int(ranges);
+    return run;
 }
 
 // How the prefill of a packed or paged batch (max_seqlen_q > 32) with plan `p`
@@ -775,7 +821,7 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
                                                                                hipStream_t stream) {
     const int st = varlen_split_ok(a, causal, splits, true);
     if (st != hipSuccess) return st;
-    const SplitPlan p = varlen_split_plan(*a, causal, splits);
+    SplitPlan p = varlen_split_plan(*a, causal, splits);
     // Top-left causal decode (max_seqlen_q <= 32) sees at most 32 keys, one
     // tile: the plan never splits it.  One-chunk bottom-right prefill needs
     // no merge either.
@@ -795,6 +841,7 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
         return launch_split<true, true, false, true>(
             shape, a->kv_heads, packed_prefill_run(shape, a->total_q, a->total_k, true, p, splits == 0), workspace, sp,
             stream);
+    if (splits == 0) p = packed_decode_run(shape, a->kv_heads, a->total_k, p);
     return br ? launch_split<true, true, false, true>(shape, a->kv_heads, p, workspace, sp, stream)
               : launch_split<false, true>(shape, a->kv_heads, p, workspace, sp, stream);
 }
@@ -834,6 +881,7 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
     const Fav4Args shape = paged_shape(*a);
     const bool br = causal == BOTTOM_RIGHT;
     if (shape.sq > DECODE_SQ) p = packed_prefill_run(shape, a->total_q, a->total_k, br, p, splits == 0);
+    else if (splits == 0) p = packed_decode_run(shape, a->kv_heads, a->total_k, p);
     return br ? launch_split<true, true, true, true>(shape, a->kv_heads, p, workspace, sp, stream)
               : launch_split<false, true, true>(shape, a->kv_heads, p, workspace, sp, stream);
 }

@@ -814,6 +814,7 @@ void fwd_kernel(Fav4Args a, Layout L, int tiles, int total, bool paired) {
             store_o_rows<TILE_BYTES, LSE>(st, inv, smem, uint32_t((ntiles & 1) * STAGE_BYTES + wave * DMA * 1024), ro,
                                           L.orow, wave * 32, a.sq - qw, lane);
         } else {
+            wait_vmem();
             const uint32_t obase = uint32_t(wave * 32 + col) * L.orow + half * 8;
             if (row < a.sq) {
 #pragma unroll
@@ -1137,6 +1138,201 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
     }
 }
 
+// Ragged packed or paged decode (up to 32 queries, one wave per workgroup, as
+// fwd_kernel_split's decode shape): the sequences' key tiles, laid end to end,
+// are cut into ranges of one length, one per workgroup, whatever sequences
+// they cross.  The kernel is bound by the K/V reads and ends with its last
+// workgroup: chunks cut per sequence (4096 of up to 64 tiles for the batch
+// below, two thirds of them past their sequence's keys) left the last round of
+// resident workgroups mostly idle.  32 sequences of 1k..32k keys H32 KVH8 (1.28
+// GB) 255 -> 207 us with the merge, 5.0 -> 6.2 TB/s; 8 of them 110 -> 87; 32 of
+// 6000..8192 keys 201 -> 147; 16 of 8 queries H64 KVH8 on 1k..16k 135 -> 102.
+// A fourth LDS stage (three tiles in flight) gives nothing (209 us).
+//  * tiles: 32-row q tiles of a group's row space; ranges: workgroups per
+//    (K/V head, q tile), all of them resident at once; min_tiles: the range
+//    length below which the longest sequence could meet more than sp.splits
+//    ranges.
+//  * A sequence without keys takes one empty tile, so that its rows are
+//    written; one without queries takes none.
+//  * The partials of a sequence's i-th range go to chunk i of the workspace;
+//    the range that starts a sequence writes -inf log-sums for the chunks it
+//    does not have, so the merge is the same.
+template <bool LSE, bool PAGED, bool BR>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void fwd_kernel_ranges(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int ranges, int min_tiles) {
+    constexpr int BN = 32, BM = 32, STAGES = 3, REGS = MAX_SORTED_SEQS / 64;
+    constexpr int TILE_BYTES = BN * ROW_BYTES;
+    constexpr int STAGE_BYTES = 2 * TILE_BYTES;
+    constexpr int DMA = BN / 4;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[STAGES * STAGE_BYTES];
+
+    const int lane = threadIdx.x;
+    const int col = lane & 31, half = lane >> 5;
+    const uint32_t row_bytes = uint32_t(a.heads) * ROW_BYTES;
+    const uint32_t kv_row_bytes = uint32_t(kv_heads) * ROW_BYTES;
+    const int group = a.heads / kv_heads, rows = group * a.sq;
+    const float scale2 = a.scale * LOG2E;
+    const uint32_t smem_base = lds_addr(smem);
+    const int bhs = a.batch * a.heads;
+    auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+
+    // With kv_heads a multiple of 8 each XCD (id % 8) reads its own K/V heads,
+    // and the q tiles of a range share its L2.
+    const int id = blockIdx.x, unit = id % kv_heads, rt = id / kv_heads;
+    const int w = uniform(rt / tiles), tile = uniform(rt - w * tiles), head0 = uniform(unit) * group;
+
+    // The range: tiles [g0, g1) of the batch, from tile g0 - base of sequence b.
+    auto key_tiles = [](const SeqSpan& s) { return s.sq > 0 ? max(1, (s.sk + BN - 1) / BN) : 0; };
+    int per, g0, b = 0, base = 0;
+    {
+        int n[REGS], total = 0;
+#pragma unroll
+        for (int k = 0; k < REGS; ++k) {
+            n[k] = 0;
+            if (k * 64 < a.batch) n[k] = key_tiles(seq_span<PAGED, true>(sp, min(k * 64 + lane, a.batch - 1), a.sq, a.sk));
+            if (k * 64 + lane >= a.batch) n[k] = 0;
+            total += n[k];
+        }
+        total = wave_total(total);
+        per = max((total + ranges - 1) / ranges, min_tiles);
+        if (int64_t(w) * per >= total) return;
+        g0 = w * per;
+#pragma unroll
+        for (int k = 0; k < REGS; ++k) {
+            const int end = wave_scan(n[k]);
+            const uint64_t hit = __builtin_amdgcn_ballot_w64(base + end > g0);
+            if (hit) {
+                const int l = __builtin_ctzll(hit);
+                b = k * 64 + l;
+                base += __builtin_amdgcn_readlane(end - n[k], l);
+                break;
+            }
+            base += __builtin_amdgcn_readlane(end, 63);
+        }
+    }
+    const int g1 = g0 + per;
+
+    const LdsOffsets off = lds_offsets(lane);
+    const DmaOffsets<DMA> dofs = dma_offsets<DMA>(0, lane, kv_row_bytes, kv_row_bytes);
+    const int q0 = tile * BM, row = q0 + col;                  // row of the group's row space
+    const int prow = min(row, rows - 1), qi = prow % a.sq, qhead = head0 + prow / a.sq;
+
+    for (;; ++b) {
+        const SeqSpan span = seq_span<PAGED>(sp, b, a.sq, a.sk);
+        const int sq = span.sq, sk = span.sk, ntiles = key_tiles(span);
+        const int t0 = max(0, g0 - base), t1 = min(min(ntiles, g1 - base), (sk + BN - 1) / BN);
+        if (ntiles > 0) {
+            const int split = w - base / per;
+            const int64_t krow0 = span.ktok * kv_heads + unit;
+            const char* kbase = static_cast<const char*>(a.k) + krow0 * ROW_BYTES;
+            const char* vbase = static_cast<const char*>(a.v) + krow0 * ROW_BYTES;
+            const rsrc_t rq = make_rsrc(static_cast<const char*>(a.q) + span.qtok * row_bytes, uint32_t(sq) * row_bytes);
+            const int64_t bh = int64_t(b) * a.heads + head0;
+            const int64_t prow0 = (int64_t(split) * bhs + bh) * a.sq + q0;
+            // Every q tile holds rows of query 0 and of the last query.
+            const int nfull = (BR ? max(0, sk - sq + 1) : sk) / BN;
+            const int climit = qi + sk - sq;                   // last visible key of this lane's row (BR)
+
+            RowState st;
+#pragma unroll
+            for (int db = 0; db < 4; ++db) st.o[db] = f32x16{};
+            st.m = -__builtin_inff();
+            st.lb = 0.f;
+            st.l = 0.f;
+            if (t0 < t1) {
+                // PAGED: lane l holds the page of slot page0 + l, for 64 slots at a time.
+                int pages = 0, page0 = 0;
+                auto load_pages = [&](int slot0) {
+                    page0 = slot0;
+                    const int slot = min(page0 + lane, sp.max_pages - 1);
+                    pages = min(max(sp.block_table[int64_t(b) * sp.max_pages + slot], 0), sp.num_pages - 1);
+                };
+                if constexpr (PAGED) load_pages(t0 * BN / sp.page_size);
+                auto issue = [&](int t) {
+                    const int first = min(t, t1 - 1) * BN;
+                    int64_t row0 = first;                      // the tile's first K/V row
+                    int rows_left = sk - first;                // rows the descriptor may cover
+                    if constexpr (PAGED) {
+                        const int slot = first / sp.page_size, in_page = first - slot * sp.page_size;
+                        if (slot - page0 >= 64) load_pages(slot);
+                        row0 = int64_t(__builtin_amdgcn_readlane(pages, slot - page0)) * sp.page_size + in_page;
+                        rows_left = min(rows_left, sp.page_size - in_page);
+                    }
+                    const uint32_t bytes = uint32_t(rows_left - 1) * kv_row_bytes + ROW_BYTES;
+                    const u32x4 rk = make_desc(kbase + row0 * kv_row_bytes, bytes);
+                    const u32x4 rv = make_desc(vbase + row0 * kv_row_bytes, bytes);
+                    dma_tile<DMA, TILE_BYTES, true>(rk, rv, smem_base + ((t - t0) % STAGES) * STAGE_BYTES, 0, dofs);
+                };
+                issue(t0);
+                issue(t0 + 1);
+                bf16x8 qr[8];
+                {
+                    const uint32_t qoff =
+                        uint32_t(min(qi, sq - 1)) * row_bytes + uint32_t(qhead) * ROW_BYTES + half * 16;
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) qr[c] = load16(rq, qoff + c * 32);
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) asm volatile("" ::"v"(qr[c]));
+                }
+                auto step = [&](auto stage_c, auto masked_c, int t) {
+                    constexpr int STAGE = decltype(stage_c)::value;
+                    const unsigned char* cur = smem + STAGE * STAGE_BYTES;
+                    wait_vmem_keep<2 * DMA>();
+                    __syncthreads();
+                    issue(t + 2);
+                    attend_fused<BN, decltype(masked_c)::value, BR, LSE, BR>(cur, cur + TILE_BYTES, off, qr, st, t == t0,
+                                                                             t * BN, sk, climit, half, scale2);
+                };
+                using S0 = std::integral_constant<int, 0>;
+                using S1 = std::integral_constant<int, 1>;
+                using S2 = std::integral_constant<int, 2>;
+                using Plain = std::integral_constant<bool, false>;
+                using Masked = std::integral_constant<bool, true>;
+                int t = t0;
+                auto triples = [&](auto masked, int end) {
+                    for (; t + 2 < end; t += 3) {
+                        step(S0{}, masked, t);
+                        step(S1{}, masked, t + 1);
+                        step(S2{}, masked, t + 2);
+                    }
+                };
+                triples(Plain{}, min(t1, nfull));
+                triples(Masked{}, t1);
+                if (t < t1) step(S0{}, Masked{}, t);
+                if (t + 1 < t1) step(S1{}, Masked{}, t + 1);
+
+                const rsrc_t rp = make_rsrc(sp.o_part + prow0 * D, uint32_t(rows - q0) * D * 4);
+                const float inv = st.lb > 0.f ? 1.f / st.lb : 0.f;
+                const uint32_t pbase = uint32_t(col) * (D * 4) + half * 16;
+#pragma unroll
+                for (int db = 0; db < 4; ++db) {
+#pragma unroll
+                    for (int vg = 0; vg < 4; ++vg) {
+                        const f32x4 x = {st.o[db][vg * 4 + 0] * inv, st.o[db][vg * 4 + 1] * inv,
+                                         st.o[db][vg * 4 + 2] * inv, st.o[db][vg * 4 + 3] * inv};
+                        store16(rp, pbase + (db * 32 + vg * 8) * 4, x);
+                    }
+                }
+            }
+            if (row < rows && qi < sq) {
+                float2* lp = reinterpret_cast<float2*>(sp.lse_part) + prow0 + col;
+                const float sb = st.m + __builtin_amdgcn_logf(st.lb);
+                if (half == 0) *lp = float2{sb, LSE ? st.m + __builtin_amdgcn_logf(st.l) : sb};
+                if (t0 == 0) {                                 // then split = 0
+                    const int chunks = (base + ntiles - 1) / per - base / per + 1;
+                    for (int s = chunks + half; s < sp.splits; s += 2)
+                        lp[int64_t(s) * bhs * a.sq] = float2{-__builtin_inff(), -__builtin_inff()};
+                }
+            }
+        }
+        base += ntiles;
+        if (base >= g1 || b + 1 >= a.batch) break;
+        // Clamped prefetches have landed before the stages are used again.
+        wait_vmem();
+        __syncthreads();
+    }
+}
+
 #pragma clang diagnostic pop
 
 // Keys that the queries [q0, q0 + bm) of a sequence can see (mask 0 dense, 1
@@ -1416,22 +1612,11 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
     // tile weighs its key tiles (by_item: with few items per workgroup slot,
     // where the last ones decide) or its sequence's longest tile's (its q
     // tiles then run together, heaviest first, and share its K/V in L2).
-    // Against that order (graph-timed, causal): 24 sequences of 64..4096
+    // Larger batches: column_item, within a pair the q tiles last-to-first.
+    // The lists against that order (graph-timed, causal): 24 sequences of 64..4096
     // tokens H32 KVH8 708 -> 582 us, 64 of 100..1000 H8 69 -> 55, 4 x 2048
     // H16 105 -> 77 (by sequence 97), 8 x 4096 H8 313 -> 264 (313); 32 of
     // 1024..7168 H8 858 -> 848.
-    // Larger batches: column_item.
-    // Against that order (graph-timed, causal): 24 sequences of 64..4096
-    // tokens H32 KVH8 708 -> 582 us, 64 of 100..1000 H8 69 -> 55, 4 x 2048
-    // H16 105 -> 77 (by sequence 97), 8 x 4096 H8 313 -> 264 (313); 32 of
-    // 1024..7168 H8 858 -> 848.
-    // Larger batches: each XCD gets a contiguous run of logical items (all q
-    // tiles of a (sequence, head) together, for its L2), but the runs are cut
-    // from the (sequence, head) pairs taken column by column from an 8-wide
-    // grid, bh = 8*row + col: XCD x holds mostly the pairs with bh % 8 == x,
-    // i.e. a share of every sequence rather than a few whole sequences, so
-    // ragged lengths do not leave XCDs idle.  Within a pair the q tiles run
-    // last-to-first (causal: heaviest first).
     const bool sorted = a.batch <= MAX_SORTED_SEQS;
     {
         const int id = int(blockIdx.y * gridDim.x + blockIdx.x);

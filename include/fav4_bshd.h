@@ -190,8 +190,10 @@ extern "C" int fav4_bshd_forward_varlen(const Fav4VarlenArgs* args, int causal, 
 //  * splits: 0 = library choice (the chunk size the contiguous split-KV Auto
 //    plan gives at the mean key length total_k / batch, at most 64 key tiles
 //    when that mean is below 3/4 of max_seqlen_k, enlarged so that the
-//    longest sequence needs at most 256 chunks), else 1..256 chunks of the
-//    longest sequence (clamped to its key tiles);
+//    longest sequence needs at most 256 chunks; a decode batch of unequal
+//    lengths and enough keys is instead cut into equal ranges of its
+//    sequences' key tiles laid end to end, within that plan's workspace),
+//    else 1..256 chunks of the longest sequence (clamped to its key tiles);
 //  * workspace as for fav4_bshd_forward_splitkv, of
 //    fav4_bshd_splitkv_varlen_workspace_size() bytes;
 //  * (heads / kv_heads) * max_seqlen_q < 2^23.

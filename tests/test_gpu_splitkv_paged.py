@@ -432,3 +432,59 @@ def test_paged_prefill_chunks(gpu_runner, case):
         seen = torch.isfinite(whole_lse)
         assert torch.equal(torch.isfinite(lse), seen) and torch.equal(torch.isfinite(lse3), seen)
         assert (lse[seen] - whole_lse[seen]).abs().max().item() <= 2e-4, splits
+
+
+# (heads, kv_heads, page_size, [(sq, sk), ...], causal): ragged decode batches
+# whose Auto takes equal ranges of the batch's keys (8 key tiles or more for
+# each of 512 workgroups): ranges that cross sequences of one key tile, none,
+# without queries and at the tile edges; more sequences than a wave's lanes;
+# bottom-right rows without a visible key; two 32-row q tiles; a range over
+# more than 64 pages.
+RANGE_CASES = [
+    (8, 8, 32, [(1, 9000), (1, 33), (0, 500), (1, 0), (1, 32), (1, 5000), (1, 31), (1, 1), (1, 2100)], 0),
+    (16, 4, 64, [(1, 37 + 997 * i % 1200) for i in range(150)], 0),
+    (32, 8, 64, [(4, 3), (4, 6001), (1, 64), (3, 0), (4, 4095), (2, 1), (4, 4097), (0, 0), (4, 3000)], 2),
+    (32, 2, 128, [(4, 30000), (2, 20001), (4, 2), (1, 12900), (4, 8200)], 2),
+    (16, 1, 32, [(1, 100), (8, 200000), (8, 8), (5, 90001)], 0),
+]
+
+
+@pytest.mark.parametrize("case", RANGE_CASES, ids=lambda c: "h%dkv%d_p%d_n%d_m%d" % (*c[:3], len(c[3]), c[4]))
+def test_ragged_decode_ranges(gpu_runner, case):
+    """Auto decode of ragged batches, paged and packed, on a workspace full of
+    NaN: within the reference bar (0.01 + 0.01 |ref|, LSE 2e-4) of the same
+    call with an explicit chunk count, rows without a key O = 0 and
+    LSE = -inf, nothing written past O, LSE and the workspace."""
+    import torch
+    h, kvh, ps, lens, causal = case
+    q, k, v, kc, vc, cu_q, cu_k, seqlens_k, table = _build(h, kvh, ps, lens, seed=131)
+    dev = torch.device("cuda:0")
+    qd, kd, vd, kcd, vcd = (to_device(x, dev) for x in (q, k, v, kc, vc))
+    cq, ck, sk_d, tb = (torch.from_numpy(x).to(dev) for x in (cu_q, cu_k, seqlens_k, table))
+    max_q, max_k, tq = max(s for s, _ in lens), max(s for _, s in lens), len(q)
+    sizes = (len(lens), h, kvh, max_q, max_k, tq, len(k))
+    print(f"  ragged decode h{h} kv{kvh} n{len(lens)} causal {causal}", flush=True)
+    _, _, ref, ref_lse = _out(torch, dev, tq, h, True)
+    gpu_runner.call_splitkv_paged(qd, kcd, vcd, ref, ref_lse, cq, sk_d, tb, max_q, max_k, 5, total_k=len(k),
+                                  causal=causal)
+    for paged in (True, False):
+        need = gpu_runner.splitkv_paged_workspace_size(*sizes, ps, table.shape[1], len(kc), 0, causal=causal) \
+            if paged else gpu_runner.splitkv_varlen_workspace_size(*sizes, causal, 0)
+        ws = torch.full((need // 4 + GUARD,), float("nan"), device=dev, dtype=torch.float32)
+        for with_lse in (True, False):
+            ob, lb, o, lse = _out(torch, dev, tq, h, with_lse)
+            if paged:
+                gpu_runner.call_splitkv_paged(qd, kcd, vcd, o, lse, cq, sk_d, tb, max_q, max_k, 0, workspace=ws,
+                                              total_k=len(k), causal=causal)
+            else:
+                gpu_runner.call_splitkv_varlen(qd, kd, vd, o, lse, cq, ck, max_q, max_k, causal, 0, workspace=ws)
+            torch.cuda.synchronize()
+            assert torch.isnan(ob[tq:]).all().item() and torch.isnan(lb[h * tq if with_lse else 0:]).all().item()
+            assert torch.isnan(ws[need // 4:]).all().item()
+            assert ((o.float() - ref.float()).abs() <= 0.01 + 0.01 * ref.float().abs()).all().item(), (paged, with_lse)
+            if with_lse:
+                seen = torch.isfinite(ref_lse)
+                assert torch.equal(torch.isfinite(lse), seen) and torch.isneginf(lse[~seen]).all().item()
+                assert (lse[seen] - ref_lse[seen]).abs().max().item() <= 2e-4, paged
+            empty = torch.isneginf(ref_lse).T
+            assert (o[empty].float() == 0).all().item()
