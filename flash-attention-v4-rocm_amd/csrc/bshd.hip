@@ -249,6 +249,31 @@ SplitPlan split_plan(const Fav4Args& a, int kv_heads, int causal, int req, bool 
     return {(ktiles + tps - 1) / tps, tps, sh, tiles, items};
 }
 
+// The chunks that Auto runs of a decode plan `p` (which sizes the workspace and
+// is what the select calls report): equal chunks run side by side, so a second
+// round of a few of them costs as much as the first, and no more are taken than
+// fit at once (H32 KVH8, graph-timed, by workgroups: B5 Sk16384 800 -> 760
+// 73.7 -> 56.8 us, B13 Sk30000 832 -> 728 294 -> 247, B7 Sk8192 784 -> 728
+// 54.1 -> 42.9, B11 Sk4096 792 -> 704 42.7 -> 36.1).  Where that makes 32
+// chunks or more of each row, two workgroups per CU do: the merge of three
+// costs more than they gain (768 and 512: B1 Sk65536 50.0 and 47.9, B2 Sk8192
+// 18.9 and 16.9, B2 Sk50000 71.6 and 68.7; B4 Sk4096, 24 and 16 chunks of a
+// row, 17.6 and 19.3, B4 Sk16384 46.9 and 49.3).  Never one chunk: that would
+// be the unpacked forward, a stream per query head.  max_tps: key tiles a
+// chunk may span.
+SplitPlan decode_run(const Fav4Args& a, const SplitPlan& p, int max_tps = INT_MAX) {
+    if (p.shape.bm != 32 || p.splits <= 2) return p;
+    const int64_t ktiles = (int64_t(a.sk) + p.shape.bn - 1) / p.shape.bn;
+    const int64_t cus = device_cus(), units = p.items * p.tiles, two = cus * 2 / units;
+    int64_t splits = two >= 32 ? two : std::max<int64_t>(2, cus * p.shape.wgs_per_cu / units);
+    splits = std::max(splits, (ktiles + max_tps - 1) / max_tps);
+    if (splits >= p.splits) return p;
+    SplitPlan run = p;
+    run.tps = int((ktiles + splits - 1) / splits);
+    run.splits = int((ktiles + run.tps - 1) / run.tps);
+    return run;
+}
+
 int64_t split_workspace(const Fav4Args& a, const SplitPlan& p) {
     if (p.splits <= 1) return 0;
     return int64_t(p.splits) * a.batch * a.heads * a.sq * (fav4::D * 4 + 2 * 4);
@@ -465,8 +490,8 @@ SplitPlan packed_split_plan(const Fav4Args& a, int kv_heads, int64_t total_k, in
 // How Auto runs the decode of a packed or paged batch whose plan is `p` (which
 // sizes the workspace): equal ranges of the batch's keys, RANGE_WGS_PER_CU
 // one-wave workgroups per CU (fwd_kernel_ranges), unless
-//  * every sequence has the longest one's keys (the contiguous plan cuts those
-//    evenly, and its result is kept bitwise);
+//  * every sequence has the longest one's keys (the contiguous call's chunks
+//    then, and its result bitwise);
 //  * a range would be under MIN_RANGE_TILES key tiles: the short ranges' fixed
 //    cost then outweighs their balance (H32 KVH8, plan / ranges: 8.5 tiles, 32
 //    sequences of 64..2048 keys 28.5 / 26.2 us; 4.1 tiles, 3 of 2500..3000
@@ -481,8 +506,10 @@ SplitPlan packed_split_plan(const Fav4Args& a, int kv_heads, int64_t total_k, in
 // 16 of 8 queries H64 on 1k..16k 102 and 115; 8 of 1k..32k 87 and 86.
 constexpr int RANGE_WGS_PER_CU = 2;
 constexpr int MIN_RANGE_TILES = 8;
-SplitPlan packed_decode_run(const Fav4Args& a, int kv_heads, int64_t total_k, const SplitPlan& p) {
-    if (a.batch > fav4::MAX_SORTED_SEQS || p.splits < 2 || total_k >= int64_t(a.batch) * a.sk) return p;
+SplitPlan packed_decode_run(const Fav4Args& a, int kv_heads, int64_t total_k, const SplitPlan& p,
+                            int max_tps = INT_MAX) {
+    if (total_k >= int64_t(a.batch) * a.sk) return decode_run(a, p, max_tps);
+    if (a.batch > fav4::MAX_SORTED_SEQS || p.splits < 2) return p;
     const int64_t streams = int64_t(kv_heads) * p.tiles;
     const int64_t ranges = int64_t(device_cus()) * RANGE_WGS_PER_CU / streams;
     if (ranges < 2) return p;
@@ -774,11 +801,12 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
                                                                             hipStream_t stream) {
     const int st = split_args_ok(a, kv_heads, causal, splits);
     if (st != hipSuccess) return st;
-    const SplitPlan p = split_plan(*a, kv_heads, causal, splits);
+    SplitPlan p = split_plan(*a, kv_heads, causal, splits);
     if (p.splits == 1) return fav4_bshd_forward_gqa(a, kv_heads, causal, 0, stream);
     const int64_t need = split_workspace(*a, p);
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255) || uint64_t(need) > workspace_bytes)
         return hipErrorInvalidValue;
+    if (splits == 0) p = decode_run(*a, p);
     const fav4::SplitArgs sp{};
     return causal ? launch_split<true>(*a, kv_heads, p, workspace, sp, stream)
                   : launch_split<false>(*a, kv_heads, p, workspace, sp, stream);
@@ -881,7 +909,7 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
     const Fav4Args shape = paged_shape(*a);
     const bool br = causal == BOTTOM_RIGHT;
     if (shape.sq > DECODE_SQ) p = packed_prefill_run(shape, a->total_q, a->total_k, br, p, splits == 0);
-    else if (splits == 0) p = packed_decode_run(shape, a->kv_heads, a->total_k, p);
+    else if (splits == 0) p = packed_decode_run(shape, a->kv_heads, a->total_k, p, PAGED_MAX_TPS);
     return br ? launch_split<true, true, true, true>(shape, a->kv_heads, p, workspace, sp, stream)
               : launch_split<false, true, true>(shape, a->kv_heads, p, workspace, sp, stream);
 }
@@ -923,9 +951,10 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_splitkv_
                                                                                     hipStream_t stream) {
     const int st = split_args_ok(a, kv_heads, causal, splits);
     if (st != hipSuccess) return st;
-    const SplitPlan p = split_plan(*a, kv_heads, causal, splits);
+    SplitPlan p = split_plan(*a, kv_heads, causal, splits);
     if (p.splits == 1) return fav4_bshd_forward_gqa(a, kv_heads, causal, 0, stream);
     if (split_workspace(*a, p) > int64_t(SCRATCH_BYTES)) return hipErrorInvalidValue;
+    if (splits == 0) p = decode_run(*a, p);
     void* ws = nullptr;
     const hipError_t e = scratch_address(&ws);
     if (e != hipSuccess) return e;

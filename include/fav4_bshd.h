@@ -76,7 +76,9 @@ extern "C" int fav4_bshd_forward_splitkv(const Fav4Args* args, int causal, int s
 // Workspace bytes fav4_bshd_forward_splitkv needs for these arguments and
 // `splits` (0 when it needs none), or -1 for rejected arguments.
 extern "C" long long fav4_bshd_splitkv_workspace_size(const Fav4Args* args, int causal, int splits);
-// The chunk count that splits = 0 resolves to (1 = no split), or -1.
+// The chunk count that splits = 0 resolves to (1 = no split), or -1.  It sizes
+// the workspace; decode (Sq <= 32) runs fewer where its workgroups would not
+// all be resident at once.
 extern "C" int fav4_bshd_splitkv_select(const Fav4Args* args, int causal);
 
 // Split-KV with grouped K/V heads (GQA / MQA); no counterpart in the

@@ -191,3 +191,48 @@ def test_splitkv_gqa(gpu_runner, shape):
                 om, lsem = _run(gpu_runner, torch, q, ke, ve, causal, splits, True)
                 assert np.array_equal(o, om), (causal, "O differs from MHA on repeated heads")
                 assert np.array_equal(lse.view(np.int32), lsem.view(np.int32)), (causal, "LSE differs")
+
+
+@pytest.mark.parametrize("shape,chunks", [((5, 32, 8, 1, 4096), 19), ((2, 32, 8, 1, 8192), 32), ((4, 32, 8, 1, 4100), 22), ((13, 8, 8, 4, 2000), 7),
+                                          ((96, 4, 4, 3, 1000), 2), ((3, 16, 8, 1, 90), 1)])
+def test_splitkv_decode_auto_chunks(gpu_runner, shape, chunks):
+    """The chunks that Auto runs of a decode call (at most as many as 768
+    one-wave workgroups, or 512 where that makes 32 of a row), bitwise the
+    explicit count's; the call without a workspace and the packed and paged
+    ones of equal lengths the same."""
+    import torch
+    b, h, kvh, sq, sk = shape
+    q, k, v = (to_device(x, torch.device("cuda:0")) for x in orc.make_inputs(b, h, sq, sk, "normal", seed=71))
+    k, v = (x[:, :, :kvh].contiguous() for x in (k, v))
+    print(f"  splitkv decode auto {shape} -> {chunks}", flush=True)
+    outs = []
+    for call in ("auto", "explicit", "noalloc", "packed", "paged"):
+        o = torch.full_like(q, float("nan"))
+        lse = torch.full((b, h, sq), float("nan"), device="cuda", dtype=torch.float32)
+        if call == "noalloc":
+            gpu_runner.call_splitkv_noalloc(q, k, v, o, lse, False, 0)
+        elif call in ("packed", "paged"):
+            if chunks == 1:
+                continue
+            cu_q = torch.arange(b + 1, device="cuda", dtype=torch.int32) * sq
+            flat = lambda x: x.reshape(-1, x.shape[2], 128)
+            packed_lse = torch.full((h, b * sq), float("nan"), device="cuda", dtype=torch.float32)
+            if call == "packed":
+                gpu_runner.call_splitkv_varlen(flat(q), flat(k), flat(v), flat(o), packed_lse, cu_q, cu_q // sq * sk,
+                                               sq, sk, False, 0)
+            else:
+                ps = 32
+                pages = -(-sk // ps)
+                pad = lambda x: torch.nn.functional.pad(x, (0, 0, 0, 0, 0, pages * ps - sk)).reshape(-1, ps, kvh, 128)
+                table = torch.arange(b * pages, device="cuda", dtype=torch.int32).reshape(b, pages)
+                lens = torch.full((b,), sk, device="cuda", dtype=torch.int32)
+                gpu_runner.call_splitkv_paged(flat(q), pad(k), pad(v), flat(o), packed_lse, cu_q, lens, table, sq, sk,
+                                              0, total_k=b * sk)
+            lse = packed_lse.reshape(h, b, sq).transpose(0, 1).contiguous()
+        else:
+            gpu_runner.call_splitkv(q, k, v, o, lse, False, chunks if call == "explicit" else 0)
+        torch.cuda.synchronize()
+        outs.append((call, o.view(torch.int16), lse.view(torch.int32)))
+    assert not torch.isnan(outs[0][1].view(torch.bfloat16)).any().item()
+    for call, o, lse in outs[1:]:
+        assert torch.equal(o, outs[0][1]) and torch.equal(lse, outs[0][2]), call
