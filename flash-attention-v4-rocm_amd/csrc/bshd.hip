@@ -334,7 +334,7 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
     sp.lse_part = sp.o_part + int64_t(p.splits) * rows * fav4::D;
     sp.splits = p.splits;
     sp.tps = p.tps;
-    sp.bm = decode ? 0 : p.shape.bm;
+    sp.bm = p.shape.bm;
     sp.mask = BR ? 2 : CAUSAL;
     // The FP32 sums only feed an LSE output.
     if (!decode) {
@@ -375,10 +375,16 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
     const int per = p.splits <= 8 ? 1 : p.splits <= 16 ? 2 : p.splits <= 32 ? 4 : 8;
     const int64_t row_blocks = (rows * per + 7) / 8;
     const unsigned blocks = unsigned(row_blocks < MAX_GRID ? row_blocks : MAX_GRID);
-    if (per == 1) hipLaunchKernelGGL((fav4::combine_kernel<1, VARLEN>), dim3(blocks), dim3(256), 0, stream, a, sp);
-    else if (per == 2) hipLaunchKernelGGL((fav4::combine_kernel<2, VARLEN>), dim3(blocks), dim3(256), 0, stream, a, sp);
-    else if (per == 4) hipLaunchKernelGGL((fav4::combine_kernel<4, VARLEN>), dim3(blocks), dim3(256), 0, stream, a, sp);
-    else hipLaunchKernelGGL((fav4::combine_kernel<8, VARLEN>), dim3(blocks), dim3(256), 0, stream, a, sp);
+    auto merge = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, stream, a, sp); };
+    auto merge_rows = [&](auto decode_c) {
+        constexpr bool DECODE = decltype(decode_c)::value;
+        if (per == 1) merge(fav4::combine_kernel<1, VARLEN, DECODE>);
+        else if (per == 2) merge(fav4::combine_kernel<2, VARLEN, DECODE>);
+        else if (per == 4) merge(fav4::combine_kernel<4, VARLEN, DECODE>);
+        else merge(fav4::combine_kernel<8, VARLEN, DECODE>);
+    };
+    if (decode) merge_rows(std::true_type{});
+    else merge_rows(std::false_type{});
     return hipGetLastError();
 }
 
