@@ -306,12 +306,12 @@ void launch_chunks(const Fav4Args& a, int kv_heads, const SplitPlan& p, const fa
     const int tiles = (a.sq + WAVES * 32 - 1) / (WAVES * 32);
     int key_bits = 1;
     while (p.tps >> key_bits) ++key_bits;
-    if (a.lse)
-        hipLaunchKernelGGL((fav4::fwd_kernel_chunk<CAUSAL, true, WAVES, KV, BR, STAGES>), item_grid(total), dim3(WAVES * 64),
-                           0, stream, a, sp, kv_heads, tiles, int(total), key_bits);
-    else
-        hipLaunchKernelGGL((fav4::fwd_kernel_chunk<CAUSAL, false, WAVES, KV, BR, STAGES>), item_grid(total), dim3(WAVES * 64),
-                           0, stream, a, sp, kv_heads, tiles, int(total), key_bits);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, item_grid(total), dim3(WAVES * 64), 0, stream, a, sp, kv_heads, tiles, int(total),
+                           key_bits);
+    };
+    if (a.lse) go(fav4::fwd_kernel_chunk<CAUSAL, true, WAVES, KV, BR, STAGES>);
+    else go(fav4::fwd_kernel_chunk<CAUSAL, false, WAVES, KV, BR, STAGES>);
 }
 
 // VARLEN: `a` holds the packed batch's shape (max lengths) and `sp` its
@@ -365,8 +365,8 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
             hipLaunchKernelGGL(kernel, dim3(grid), dim3(64), 0, stream, a, sp, kv_heads, tiles, int(total));
         };
         if constexpr (!CAUSAL || BR) {
-            if (a.lse) go(fav4::fwd_kernel_split<32, BR, 1, true, VARLEN, PAGED, BR>);
-            else go(fav4::fwd_kernel_split<32, BR, 1, false, VARLEN, PAGED, BR>);
+            if (a.lse) go(fav4::fwd_kernel_split<true, VARLEN, PAGED, BR>);
+            else go(fav4::fwd_kernel_split<false, VARLEN, PAGED, BR>);
         }
     }
     const hipError_t e = hipGetLastError();

@@ -59,8 +59,9 @@ __host__ __device__ constexpr int items_per_head(int tiles, bool paired) { retur
 
 template <bool CAUSAL, class F>
 __device__ __forceinline__ void for_item(int tiles, int total, bool paired, F&& process) {
-    const int id = int(blockIdx.y * gridDim.x + blockIdx.x);
-    if (id >= total) return;
+    const uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;      // may pass INT_MAX in the last row
+    if (wg >= uint32_t(total)) return;
+    const int id = int(wg);
     const int per_head = items_per_head(tiles, CAUSAL && paired);
     const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
     const int logical = xcd * per + min(xcd, rem) + slot;
@@ -91,10 +92,11 @@ struct Span {
 // shortest, and nothing is launched for the q tiles that a shorter sequence
 // does not have.  A sequence has `tiles` items; those that weigh c or more are
 // all of them while (c - 1) * UNIT < keys, less one for every BM by which
-// (c - 1) * UNIT passes `shift` (c = 0: all).  Each wave finds item `rank` by itself, the
-// sequences (up to 4 * 64) in its lanes: a binary search for the weight, of
-// key_bits bits, whose items hold `rank`, then one scan over the sequences
-// (some 200 instructions, about 0.6 us against 8 us and more for an item).
+// (c - 1) * UNIT passes `shift` (c = 0: all).  Each wave finds item `rank` by
+// itself, the sequences (up to 4 * 64) in its lanes: a binary search for the
+// weight, of key_bits bits, whose items hold `rank`, then one scan over the
+// sequences (some 200 instructions, about 0.6 us against 8 us and more for an
+// item).
 // Returns the sequence, its span and the item's place among that sequence's
 // (0 = its heaviest); seq = -1 past the last item.
 constexpr int MAX_SORTED_SEQS = 256;
@@ -873,15 +875,14 @@ struct SplitArgs {
     const int* block_table;
     int page_size, max_pages, num_pages;
     // What the merge needs to count a prefill row's chunks: query rows per q
-    // tile and the mask (0 dense, 1
-    // top-left, 2 bottom-right).
+    // tile and the mask (0 dense, 1 top-left, 2 bottom-right).
     int bm, mask;
 };
 
 // Query / key count and first token of sequence b (the same in every lane of
-// the workgroup unless PER_LANE), read on the device and clamped to [0, total] and to the max
-// lengths, as fwd_kernel_varlen does.  PAGED: the key count is seqlens_k[b]
-// clamped to [0, max_k] (ktok unused).
+// the workgroup unless PER_LANE), read on the device and clamped to [0, total]
+// and to the max lengths, as fwd_kernel_varlen does.  PAGED: the key count is
+// seqlens_k[b] clamped to [0, max_k] (ktok unused).
 struct SeqSpan {
     int sq, sk;
     int64_t qtok, ktok;
@@ -897,48 +898,41 @@ __device__ __forceinline__ SeqSpan seq_span(const SplitArgs& sp, int b, int max_
     return {qe - qs, ke - ks, qs, ks};
 }
 
-// Three LDS stages keep two key tiles in flight per workgroup (prefetch
-// distance 2).  Long-key prefill chunks run as fast as with two; decode-like
-// chunks, where one wave computes and the kernel mostly streams K/V, gain up
-// to 10% (measured), since the DMA latency rather than the MFMAs bounds a tile.
-// WAVES = 8, BN = 64: long-key prefill chunks (256-row q tiles).  WAVES = 1,
-// BN = 32: decode (sq <= 32): one wave per workgroup and 48 KiB of LDS, so
-// three workgroups share a CU and every resident wave computes.
+// Decode chunks (sq <= 32): one wave per workgroup, 32-key tiles and 48 KiB of
+// LDS, so three workgroups share a CU and every resident wave computes.  Three
+// LDS stages keep two key tiles in flight (prefetch distance 2), up to 10%
+// faster than one, since the DMA latency rather than the MFMAs bounds a tile.
 // LSE: keep the FP32 sums for the LSE output; without it the second log-sum
 // repeats the first (the merge reads it only when writing an LSE).
 // VARLEN: packed sequences; a.sq / a.sk are the max lengths, rows keep the
 // a.sq stride, and rows past a sequence's own length are computed on a valid
-// query but never read by the merge (eight waves: q tiles past them exit).
+// query but never read by the merge.
 // PAGED (with VARLEN): K/V come from paged caches.  page_size is a multiple
-// of BN, so a key tile lies in one page; a chunk spans at most 64 pages, whose
+// of 32, so a key tile lies in one page; a chunk spans at most 64 pages, whose
 // (clamped) numbers one load puts in the wave's lanes at the chunk start.
-// BR (with CAUSAL and VARLEN): bottom-right causal, query i of a sequence
+// BR (with VARLEN): bottom-right causal, query i of a sequence
 // with sq queries and sk keys sees keys j <= sk - sq + i (the last query sees
 // all of them; with sq > sk the first sq - sk rows see none).
-// The one-wave shape keeps the 8-wave shape's 256-register budget
-// (waves_per_eu 2); its occupancy is set by LDS (three workgroups per CU), so
-// the compiler's note that it cannot reach two waves per SIMD is expected.
+// It keeps the prefill kernels' 256-register budget (waves_per_eu 2); its
+// occupancy is set by LDS (three workgroups per CU), so the compiler's note
+// that it cannot reach two waves per SIMD is expected.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
-template <int BN, bool CAUSAL, int WAVES, bool LSE, bool VARLEN = false, bool PAGED = false, bool BR = false>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <bool LSE, bool VARLEN = false, bool PAGED = false, bool BR = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int total) {
     static_assert(!PAGED || VARLEN, "paged caches hold packed sequences");
-    static_assert(!BR || (CAUSAL && VARLEN), "bottom-right causal needs per-sequence lengths");
-    constexpr int BM = WAVES * 32, STAGES = 3;
-    // One wave (decode): the q-tile rows are the group's query heads times
-    // their sq queries, row r = (head - first head of the group) * sq + query,
-    // so the heads that share a K/V head stream it once.  Eight waves: the
-    // rows of one head.
-    constexpr bool PACK = WAVES == 1;
+    static_assert(!BR || VARLEN, "bottom-right causal needs per-sequence lengths");
+    // The q-tile rows are the group's query heads times their sq queries, row
+    // r = (head - first head of the group) * sq + query, so the heads that
+    // share a K/V head stream it once.
+    constexpr int BN = 32, BM = 32, STAGES = 3;
     constexpr int TILE_BYTES = BN * ROW_BYTES;
     constexpr int STAGE_BYTES = 2 * TILE_BYTES;
-    constexpr int DMA = BN / 4 / WAVES;
-    static_assert(BN % 32 == 0 && BN % (4 * WAVES) == 0, "tile shape");
+    constexpr int DMA = BN / 4;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[STAGES * STAGE_BYTES];
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x;
     const int col = lane & 31, half = lane >> 5;
     const uint32_t row_bytes = uint32_t(a.heads) * ROW_BYTES;
     const uint32_t kv_row_bytes = uint32_t(kv_heads) * ROW_BYTES;
@@ -948,15 +942,13 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
     const int bhs = a.batch * a.heads;
 
     const LdsOffsets off = lds_offsets(lane);
-    const DmaOffsets<DMA> dofs = dma_offsets<DMA>(wave, lane, kv_row_bytes, kv_row_bytes);
+    const DmaOffsets<DMA> dofs = dma_offsets<DMA>(0, lane, kv_row_bytes, kv_row_bytes);
 
-    // Rows of one item's row space: a head's queries, or a group's.
-    const int rows = PACK ? group * a.sq : a.sq;
-    const int items_per_batch = PACK ? kv_heads : a.heads;
-    const int npairs = a.batch * items_per_batch, full = npairs >> 3, rem8 = npairs & 7;
+    const int rows = group * a.sq;                             // of one item's row space
+    const int npairs = a.batch * kv_heads, full = npairs >> 3, rem8 = npairs & 7;
     for (int id = blockIdx.x; id < total; id += gridDim.x) {
-        // XCD-contiguous order; within a (b, h) -- PACK: (b, K/V head) -- the
-        // q tiles of one key chunk are adjacent, so they share it in L2.
+        // XCD-contiguous order; within a (b, K/V head) the q tiles of one key
+        // chunk are adjacent, so they share it in L2.
         const int xcd = id & 7, slot = id >> 3, per = total >> 3, rem = total & 7;
         const int logical = xcd * per + min(xcd, rem) + slot;
         const int per_item = tiles * sp.splits;
@@ -965,7 +957,7 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
         if constexpr (VARLEN) {
             // Packed sequences differ in length: take the (sequence, head)
             // pairs column by column from an 8-wide grid (it = 8 * row + col,
-            // as fwd_kernel_varlen does), so XCD x works on the pairs with
+            // as column_item does), so XCD x works on the pairs with
             // it % 8 == x -- a share of every sequence -- instead of a few
             // whole sequences.  With 8 K/V heads each XCD gets one head of
             // every sequence.
@@ -983,13 +975,12 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
         }
         const int split = r / tiles, tile = r - split * tiles;
 
-        // it = b*heads + h, or (PACK) b*kv_heads + K/V head; head0 = the first
-        // query head of the item's rows.
-        const int batch = it / items_per_batch, unit = it - batch * items_per_batch;
-        const int head0 = PACK ? unit * group : unit;
+        // it = b*kv_heads + K/V head; head0 = the first query head of its rows.
+        const int batch = it / kv_heads, unit = it - batch * kv_heads;
+        const int head0 = unit * group;
         const int bh = batch * a.heads + head0;
-        const int q0 = tile * BM, qw = q0 + wave * 32;
-        const int row = qw + col;                              // row of the item's row space
+        const int q0 = tile * BM;
+        const int row = q0 + col;                              // row of the item's row space
         // The sequence: its query / key counts and first tokens.
         SeqSpan span{a.sq, a.sk, int64_t(batch) * a.sq, int64_t(batch) * a.sk};
         // PAGED: lane l holds the page of the chunk's l-th page slot, loaded
@@ -1001,18 +992,17 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
         }
         if constexpr (VARLEN) {
             span = seq_span<PAGED>(sp, batch, a.sq, a.sk);
-            // No query rows (eight waves: none from this q tile on): nothing to merge.
-            if (span.sq == 0 || (!PACK && q0 >= span.sq)) continue;
+            if (span.sq == 0) continue;                        // no query rows: nothing to merge
         }
         const int sq = span.sq, sk = span.sk;
         // This lane's query position (causal limit) and Q byte offset inside
         // the sequence's [sq, heads] block; rows past the space (or past the
         // sequence's queries) read a valid row.
         const int prow = min(row, rows - 1);
-        const int qi = PACK ? prow % a.sq : prow;
-        const int qhead = PACK ? head0 + prow / a.sq : head0;
+        const int qi = prow % a.sq;
+        const int qhead = head0 + prow / a.sq;
         const int qload = min(qi, sq - 1);
-        const int64_t krow0 = span.ktok * kv_heads + head0 / group;
+        const int64_t krow0 = span.ktok * kv_heads + unit;
         const char* kbase = static_cast<const char*>(a.k) + krow0 * ROW_BYTES;
         const char* vbase = static_cast<const char*>(a.v) + krow0 * ROW_BYTES;
         const rsrc_t rq = make_rsrc(static_cast<const char*>(a.q) + span.qtok * row_bytes, uint32_t(sq) * row_bytes);
@@ -1020,18 +1010,12 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
         // group's heads are adjacent, so its rows are contiguous).
         const int64_t prow0 = (int64_t(split) * bhs + bh) * a.sq + q0;
         const rsrc_t rp = make_rsrc(sp.o_part + prow0 * D, uint32_t(rows - q0) * D * 4);
-        // PACK: every q tile holds rows of query 0 and of the last query, so
-        // the causal range is the whole [0, min(sk, sq)) and no tile is
-        // unmasked for every row.  BR: unmasked for every row below key
-        // sk - sq + 1 (query 0's first hidden key); PACK sees [0, sk) (its
-        // tile holds the last query), a q tile of rows [q0, q0 + BM) only up
-        // to its last row's diagonal, so chunks past it are empty.
-        const int kend = !CAUSAL ? sk
-                         : BR    ? (PACK ? sk : min(sk, max(0, min(sq, q0 + BM) + sk - sq)))
-                                 : min(sk, PACK ? sq : q0 + BM);
-        const int ntiles = (kend + BN - 1) / BN;
-        const int nfull = (BR ? max(0, (PACK ? 0 : q0) + sk - sq + 1) : CAUSAL ? (PACK ? 0 : min(sk, q0 + 1)) : sk) / BN;
-        const int climit = BR ? qi + sk - sq : qi;     // last visible key of this lane's row
+        // Every q tile holds rows of query 0 and of the last query.  BR: tiles
+        // are unmasked for every row below key sk - sq + 1 (query 0's first
+        // hidden key).
+        const int ntiles = (sk + BN - 1) / BN;
+        const int nfull = (BR ? max(0, sk - sq + 1) : sk) / BN;
+        const int climit = qi + sk - sq;                       // last visible key of this lane's row (BR)
         const int t0 = split * sp.tps, t1 = min(ntiles, t0 + sp.tps);
 
         RowState st;
@@ -1059,7 +1043,7 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
                 const uint32_t bytes = uint32_t(rows_left - 1) * kv_row_bytes + ROW_BYTES;
                 const u32x4 rk = make_desc(kbase + row0 * kv_row_bytes, bytes);
                 const u32x4 rv = make_desc(vbase + row0 * kv_row_bytes, bytes);
-                dma_tile<DMA, TILE_BYTES, PACK>(rk, rv, smem_base + ((t - t0) % STAGES) * STAGE_BYTES, wave, dofs);
+                dma_tile<DMA, TILE_BYTES, true>(rk, rv, smem_base + ((t - t0) % STAGES) * STAGE_BYTES, 0, dofs);
             };
             issue(t0);
             issue(t0 + 1);
@@ -1071,18 +1055,15 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
 #pragma unroll
                 for (int c = 0; c < 8; ++c) asm volatile("" ::"v"(qr[c]));
             }
-            // Wait for tile t (tile t+1 may stay in flight), then prefetch
-            // tile t+2 into the stage freed by the barrier (tile t-1's).
-            auto sync_and_prefetch = [&](int t) {
-                wait_vmem_keep<2 * DMA>();
-                __syncthreads();
-                issue(t + 2);
-            };
             auto step = [&](auto stage_c, auto masked_c, int t) {
                 constexpr int STAGE = decltype(stage_c)::value;
                 const unsigned char* cur = smem + STAGE * STAGE_BYTES;
-                sync_and_prefetch(t);
-                attend_fused<BN, decltype(masked_c)::value, CAUSAL, LSE, CAUSAL>(
+                // Wait for tile t (tile t+1 may stay in flight), then prefetch
+                // tile t+2 into the stage freed by the barrier (tile t-1's).
+                wait_vmem_keep<2 * DMA>();
+                __syncthreads();
+                issue(t + 2);
+                attend_fused<BN, decltype(masked_c)::value, BR, LSE, BR>(
                     cur, cur + TILE_BYTES, off, qr, st, t == t0, t * BN, sk, climit, half, scale2);
             };
             using S0 = std::integral_constant<int, 0>;
@@ -1092,33 +1073,27 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
             using Masked = std::integral_constant<bool, true>;
             int t = t0;
             const int tp = min(t1, nfull);
-            if (qw >= (VARLEN && !PACK ? sq : rows)) {
-                // Rows all past sq (decode: 7 of 8 waves): only the DMA and
-                // barrier sequence of the loop below.
-                for (; t < t1; ++t) sync_and_prefetch(t);
-            } else {
-                for (; t + 2 < tp; t += 3) {
-                    step(S0{}, Plain{}, t);
-                    step(S1{}, Plain{}, t + 1);
-                    step(S2{}, Plain{}, t + 2);
-                }
-                // (t - t0) % 3 == 0 here: the masked tiles run in compile-time
-                // stage triples as well, so O keeps one register home.
-                for (; t + 2 < t1; t += 3) {
-                    step(S0{}, Masked{}, t);
-                    step(S1{}, Masked{}, t + 1);
-                    step(S2{}, Masked{}, t + 2);
-                }
-                if (t < t1) step(S0{}, Masked{}, t);
-                if (t + 1 < t1) step(S1{}, Masked{}, t + 1);
+            for (; t + 2 < tp; t += 3) {
+                step(S0{}, Plain{}, t);
+                step(S1{}, Plain{}, t + 1);
+                step(S2{}, Plain{}, t + 2);
             }
+            // (t - t0) % 3 == 0 here: the masked tiles run in compile-time
+            // stage triples as well, so O keeps one register home.
+            for (; t + 2 < t1; t += 3) {
+                step(S0{}, Masked{}, t);
+                step(S1{}, Masked{}, t + 1);
+                step(S2{}, Masked{}, t + 2);
+            }
+            if (t < t1) step(S0{}, Masked{}, t);
+            if (t + 1 < t1) step(S1{}, Masked{}, t + 1);
         }
 
         // Chunk epilogue: FP32 O / lb and the two log2-domain sums.  A packed
         // sequence's chunks past its keys skip the O rows: their log-sums are
         // -inf, so the merge gives them weight 0 and never adds their O.
         const float inv = st.lb > 0.f ? 1.f / st.lb : 0.f;
-        const uint32_t pbase = uint32_t(wave * 32 + col) * (D * 4) + half * 16;
+        const uint32_t pbase = uint32_t(col) * (D * 4) + half * 16;
 #pragma unroll
         for (int db = 0; db < 4 && !(VARLEN && t0 >= t1); ++db) {
 #pragma unroll
@@ -1387,8 +1362,9 @@ void fwd_kernel_chunk(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
     const int bhs = a.batch * a.heads;
 
     // The item: (sequence, head, q tile, chunk), one per workgroup.
-    const int id = int(blockIdx.y * gridDim.x + blockIdx.x);
-    if (id >= total) return;
+    const uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;
+    if (wg >= uint32_t(total)) return;
+    const int id = int(wg);
     int batch, head, unit, ntile = tiles;
     SeqSpan span;
     if constexpr (KV == 0) {
@@ -1620,8 +1596,9 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
     // 1024..7168 H8 858 -> 848.
     const bool sorted = a.batch <= MAX_SORTED_SEQS;
     {
-        const int id = int(blockIdx.y * gridDim.x + blockIdx.x);
-        if (id >= total) return;
+        const uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;
+        if (wg >= uint32_t(total)) return;
+        const int id = int(wg);
         int batch, head, tile;
         Span sp;
         if (sorted) {
