@@ -1302,9 +1302,10 @@ void fwd_kernel_ranges(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int ra
             }
         }
         base += ntiles;
-        if (base >= g1 || b + 1 >= a.batch) break;
-        // Clamped prefetches have landed before the stages are used again.
+        // Clamped prefetches have landed before the stages are used again, by
+        // the next sequence or, after the last one, by the CU's next workgroup.
         wait_vmem();
+        if (base >= g1 || b + 1 >= a.batch) break;
         __syncthreads();
     }
 }
