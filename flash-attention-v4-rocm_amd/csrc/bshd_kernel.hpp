@@ -1735,7 +1735,13 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
 // (4 dims per lane) with no branch between the loads, and the groups' partial
 // sums are added in LDS.  Many chunks over few rows (decode) thus take a few
 // memory round trips instead of one pair of dependent loads per chunk.
-// DECODE: every row merges sp.splits chunks.
+// Bound by the latency of its few loads, so by the waves that fit a SIMD: one
+// lane for each chunk's log-sums, 32-bit row arithmetic and loads that need no
+// mask of their own keep PER 1 at 59 - 70 VGPRs (7 or 8 waves; at 94 - 108, 4
+// or 5, the merge of 592k causal rows of 2 chunks took 215 - 286 us against
+// 161, of 16640 one-chunk decode rows 25 - 27 against 15) and PER 8 at two waves.
+// DECODE: every row merges sp.splits chunks.  Prefill rows merge as many as
+// they see keys of; past those, the row's last chunk is read with weight 0.
 // VARLEN: rows are (sequence, head, query < max_seqlen_q); rows past their
 // sequence's query count are skipped, O goes to the sequence's token rows and
 // LSE to [heads, total_q]; a row whose chunks saw no key gets O = 0 and
@@ -1756,7 +1762,7 @@ __device__ __forceinline__ float sum32(float x) {
 
 template <int PER, bool VARLEN, bool DECODE>
 __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) {
-    constexpr int RPB = 8 / PER, NT = PER * 32, MAXV = (MAX_SPLITS + NT - 1) / NT;
+    constexpr int RPB = 8 / PER;
     // Chunks per lane group: PER = 1, 2, 4 serve up to 8, 16, 32 chunks; 8 up to MAX_SPLITS.
     constexpr int NS = PER == 8 ? (MAX_SPLITS + 7) / 8 : 8;
     __shared__ float wsh[RPB][MAX_SPLITS];   // chunk weights 2^(lse_b,s - max)
@@ -1764,17 +1770,17 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
     __shared__ f32x4 part_acc[8][32];
     const int grp = threadIdx.x >> 5, q4 = threadIdx.x & 31;
     const int slot = grp / PER, part = grp - slot * PER;
-    const int team = part * 32 + q4;
-    const int64_t rows = int64_t(a.batch) * a.heads * a.sq;
+    const int team = part * 32 + q4;                // the chunk whose log-sums this lane reads
+    const uint32_t rows = uint32_t(a.batch) * uint32_t(a.heads) * uint32_t(a.sq);   // at most INT_MAX
     const int64_t slab = rows;                      // rows per chunk
-    const int64_t blocks = (rows + RPB - 1) / RPB;
+    const uint32_t blocks = (rows + RPB - 1) / RPB;
 
     // Workgroup-uniform loop: every wave reaches every barrier.
-    for (int64_t blk = blockIdx.x; blk < blocks; blk += gridDim.x) {
-        const int64_t r = blk * RPB + slot;
-        const int64_t bh = r / a.sq;
-        const int qi = int(r - bh * a.sq);
-        const int batch = int(bh / a.heads), head = int(bh - int64_t(batch) * a.heads);
+    for (uint32_t blk = blockIdx.x; blk < blocks; blk += gridDim.x) {
+        const uint32_t r = blk * RPB + slot;
+        const uint32_t bh = r / uint32_t(a.sq);
+        const int qi = int(r - bh * uint32_t(a.sq));
+        const int batch = int(bh / uint32_t(a.heads)), head = int(bh - uint32_t(batch) * uint32_t(a.heads));
         int64_t qtok = int64_t(batch) * a.sq + qi;       // the row's token (BSHD)
         bool live = r < rows;
         int sq = a.sq, sk = a.sk, nch = sp.splits, cu0 = 0, cu1 = 0;
@@ -1795,10 +1801,10 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
         if (!DECODE && (VARLEN || sp.mask)) {
             // A q tile of one chunk was written by it; the others have as many
             // chunks as their visible keys (BSHD dense: all have sp.splits).
-            const int vis = visible_keys(sp.mask, qi - qi % sp.bm, sp.bm, sq, sk);
-            nch = min(sp.splits, ((vis + 63) / 64 + sp.tps - 1) / sp.tps);
+            const int vis = visible_keys(sp.mask, qi & -sp.bm, sp.bm, sq, sk);
+            nch = min(sp.splits, int(uint32_t((vis + 63) / 64 + sp.tps - 1) / uint32_t(sp.tps)));
             if (nch <= 1) live = false;
-            if (!__syncthreads_or(live)) continue;
+            if (VARLEN && !__syncthreads_or(live)) continue;
         }
         // The partial O rows do not depend on the weights: their loads go out
         // first, so that their latency overlaps the log-sum phase (one memory
@@ -1807,34 +1813,29 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
         // beside the query offsets, also for the rows that its sequence turns
         // out not to have (with the chunk kernel's page numbers beside its
         // lengths, 8 sequences of 100..2000 keys 15.1 -> 14.75 us).
-        const float* op = sp.o_part + r * D + q4 * 4;
+        const float* op = sp.o_part + int64_t(r) * D + q4 * 4;
         f32x4 xo[NS];
 #pragma unroll
-        for (int i = 0; i < NS; ++i) {
-            const int s = part + i * PER;
-            xo[i] = live && s < nch ? *reinterpret_cast<const f32x4*>(op + s * slab * D) : f32x4{};
-        }
-        float vb[MAXV], vl[MAXV];
-        float mb = -__builtin_inff(), ml = -__builtin_inff();
+        for (int i = 0; i < NS; ++i) xo[i] = f32x4{};
+        if (live) {
 #pragma unroll
-        for (int i = 0; i < MAXV; ++i) {
-            const int s = team + i * NT;
-            vb[i] = vl[i] = -__builtin_inff();
-            if (live && s < nch) {
-                const float2 v = *reinterpret_cast<const float2*>(sp.lse_part + (s * slab + r) * 2);
-                vb[i] = v.x;
-                vl[i] = v.y;
+            for (int i = 0; i < NS; ++i) {
+                const int s = part + i * PER;
+                if (s < sp.splits) xo[i] = *reinterpret_cast<const f32x4*>(op + (DECODE ? s : min(s, nch - 1)) * slab * D);
             }
-            mb = fmaxf(mb, vb[i]);
-            ml = fmaxf(ml, vl[i]);
+        }
+        float vb = -__builtin_inff(), vl = -__builtin_inff();
+        if (live && team < nch) {
+            const float2 v = *reinterpret_cast<const float2*>(sp.lse_part + (team * slab + int64_t(r)) * 2);
+            vb = v.x;
+            vl = v.y;
         }
         if constexpr (VARLEN && DECODE) {
             const int qs = min(max(cu0, 0), sp.total_q);
             live = live && qi < min(max(cu1, qs), min(sp.total_q, qs + a.sq)) - qs;
             qtok = int64_t(qs) + qi;
         }
-        mb = max32(mb);
-        ml = max32(ml);
+        float mb = max32(vb), ml = max32(vl);
         if (q4 == 0) red_m[grp] = float2{mb, ml};
         __syncthreads();
 #pragma unroll
@@ -1847,15 +1848,10 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
             if (mb == -__builtin_inff()) mb = ml = 0.f;
         }
         float den = 0.f, suml = 0.f;
-#pragma unroll
-        for (int i = 0; i < MAXV; ++i) {
-            const int s = team + i * NT;
-            if (s < nch) {
-                const float w = live ? exp2_native(vb[i] - mb) : 0.f;
-                wsh[slot][s] = w;
-                den += w;
-                if (live) suml += exp2_native(vl[i] - ml);
-            }
+        if (team < sp.splits) {
+            den = live ? exp2_native(vb - mb) : 0.f;
+            wsh[slot][team] = den;
+            if (live) suml = exp2_native(vl - ml);
         }
         den = sum32(den);
         suml = sum32(suml);
@@ -1875,7 +1871,7 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
 #pragma unroll
             for (int i = 0; i < NS; ++i) {
                 const int s = part + i * PER;
-                if (s < nch) {
+                if (s < sp.splits) {
                     const float w = wsh[slot][s];
                     if (w > 0.f) acc += w * xo[i];
                 }
@@ -1897,7 +1893,7 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
             *reinterpret_cast<bf16x4*>(static_cast<char*>(a.o) + orow * ROW_BYTES + q4 * 8) =
                 bf16x4{b0[0], b0[1], b1[0], b1[1]};
             if (a.lse && q4 == 0) {
-                const int64_t li = VARLEN ? int64_t(head) * sp.total_q + qtok : r;
+                const int64_t li = VARLEN ? int64_t(head) * sp.total_q + qtok : int64_t(r);
                 a.lse[li] = (ml + __builtin_amdgcn_logf(suml)) * LN2;
             }
         }
