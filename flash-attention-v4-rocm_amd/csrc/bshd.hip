@@ -522,8 +522,9 @@ SplitPlan packed_decode_run(const Fav4Args& a, int kv_heads, int64_t total_k, co
     const int64_t ktiles = (a.sk + p.shape.bn - 1) / p.shape.bn;
     const int64_t range = (total_k / p.shape.bn + a.batch / 2 + ranges - 1) / ranges;
     if (range < MIN_RANGE_TILES || ktiles > range * (p.splits - 1)) return p;
+    const int64_t full = range + int64_t(a.batch) * fav4::RANGE_SEQ_TILES / ranges;
     SplitPlan run = p;
-    run.splits = int(std::min<int64_t>(p.splits, (ktiles + range - 1) / range + 2));
+    run.splits = int(std::min<int64_t>(p.splits, (ktiles + full - 1) / full + 2));
     run.ranges = int(ranges);
     return run;
 }

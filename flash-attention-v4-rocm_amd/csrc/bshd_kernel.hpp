@@ -1128,11 +1128,18 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
 //    (K/V head, q tile), all of them resident at once; min_tiles: the range
 //    length below which the longest sequence could meet more than sp.splits
 //    ranges.
+//  * A sequence counts RANGE_SEQ_TILES more than its key tiles, laid before
+//    them, for what its lengths, pages, queries and partials cost a range
+//    (with 0, 2, 4 and 8 of them: 63 sequences of 50 keys and one of 200000,
+//    H32 KVH8, 350, 221, 179 and 166 us; 2 of 1381 and 30000 34.3, 33.0, 30.8
+//    and 30.9; 22 of 16 queries on 153..8152, H12 KVH3, 48.9, 46.4, 43.0 and
+//    40.6).
 //  * A sequence without keys takes one empty tile, so that its rows are
 //    written; one without queries takes none.
 //  * The partials of a sequence's i-th range go to chunk i of the workspace;
 //    the range that starts a sequence writes -inf log-sums for the chunks it
 //    does not have, so the merge is the same.
+constexpr int RANGE_SEQ_TILES = 8;
 template <bool LSE, bool PAGED, bool BR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fwd_kernel_ranges(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int ranges, int min_tiles) {
@@ -1157,7 +1164,8 @@ void fwd_kernel_ranges(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int ra
     const int id = blockIdx.x, unit = id % kv_heads, rt = id / kv_heads;
     const int w = uniform(rt / tiles), tile = uniform(rt - w * tiles), head0 = uniform(unit) * group;
 
-    // The range: tiles [g0, g1) of the batch, from tile g0 - base of sequence b.
+    // The range: tiles [g0, g1) of the batch, from sequence b, whose first is
+    // number `base`.
     auto key_tiles = [](const SeqSpan& s) { return s.sq > 0 ? max(1, (s.sk + BN - 1) / BN) : 0; };
     int per, g0, b = 0, base = 0;
     {
@@ -1167,6 +1175,7 @@ void fwd_kernel_ranges(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int ra
             n[k] = 0;
             if (k * 64 < a.batch) n[k] = key_tiles(seq_span<PAGED, true>(sp, min(k * 64 + lane, a.batch - 1), a.sq, a.sk));
             if (k * 64 + lane >= a.batch) n[k] = 0;
+            if (n[k] > 0) n[k] += RANGE_SEQ_TILES;
             total += n[k];
         }
         total = wave_total(total);
@@ -1196,9 +1205,10 @@ void fwd_kernel_ranges(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int ra
     for (;; ++b) {
         const SeqSpan span = seq_span<PAGED>(sp, b, a.sq, a.sk);
         const int sq = span.sq, sk = span.sk, ntiles = key_tiles(span);
-        const int t0 = max(0, g0 - base), t1 = min(min(ntiles, g1 - base), (sk + BN - 1) / BN);
-        if (ntiles > 0) {
-            const int split = w - base / per;
+        const int first = base + RANGE_SEQ_TILES;              // its first key tile
+        const int t0 = max(0, g0 - first), t1 = min(min(ntiles, g1 - first), (sk + BN - 1) / BN);
+        if (ntiles > 0 && first < g1) {
+            const int split = w - first / per;
             const int64_t krow0 = span.ktok * kv_heads + unit;
             const char* kbase = static_cast<const char*>(a.k) + krow0 * ROW_BYTES;
             const char* vbase = static_cast<const char*>(a.v) + krow0 * ROW_BYTES;
@@ -1295,13 +1305,13 @@ void fwd_kernel_ranges(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int ra
                 const float sb = st.m + __builtin_amdgcn_logf(st.lb);
                 if (half == 0) *lp = float2{sb, LSE ? st.m + __builtin_amdgcn_logf(st.l) : sb};
                 if (t0 == 0) {                                 // then split = 0
-                    const int chunks = (base + ntiles - 1) / per - base / per + 1;
+                    const int chunks = (first + ntiles - 1) / per - first / per + 1;
                     for (int s = chunks + half; s < sp.splits; s += 2)
                         lp[int64_t(s) * bhs * a.sq] = float2{-__builtin_inff(), -__builtin_inff()};
                 }
             }
         }
-        base += ntiles;
+        if (ntiles > 0) base = first + ntiles;
         // Clamped prefetches have landed before the stages are used again, by
         // the next sequence or, after the last one, by the CU's next workgroup.
         wait_vmem();

@@ -1,0 +1,62 @@
+"""GPU checks that a batch is not slower than the parts of it that bound it.
+
+Each case compares two calls of this library on one box, timed in turn, by a
+ratio with a wide margin on both sides of what was measured.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _ratio(torch, slow, fast, calls=20, rounds=5):
+    """Time of `slow` over time of `fast`: the median of the rounds' ratios."""
+    def us(fn):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(calls):
+            fn()
+        b.record()
+        torch.cuda.synchronize()
+        return a.elapsed_time(b) * 1e3 / calls
+    us(slow), us(fast)
+    times = [(us(slow), us(fast)) for _ in range(rounds)]
+    print("  us:", *("%.1f / %.1f" % t for t in times), flush=True)
+    return float(np.median([s / f for s, f in times]))
+
+
+def _paged(torch, runner, h, kvh, lens_q, lens_k, causal=0, ps=64, splits=0, total_k=True):
+    """A paged call on its own buffers; returns the function that runs it."""
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(7)
+    mk = lambda *s: torch.randn(s, device=dev, dtype=torch.float32, generator=g).to(torch.bfloat16)
+    pages = [-(-n // ps) for n in lens_k]
+    table = torch.zeros((len(pages), max(pages)), dtype=torch.int32)
+    first = 0
+    for i, n in enumerate(pages):
+        table[i, :n] = torch.arange(first, first + n)
+        first += n
+    table = table.to(dev)
+    cu_q = torch.tensor(np.concatenate([[0], np.cumsum(lens_q)]), dtype=torch.int32, device=dev)
+    keys = torch.tensor(lens_k, dtype=torch.int32, device=dev)
+    q, kc, vc = mk(sum(lens_q), h, 128), mk(first, ps, kvh, 128), mk(first, ps, kvh, 128)
+    o = torch.empty_like(q)
+    max_q, max_k = max(lens_q), max(lens_k)
+    total = sum(lens_k) if total_k else max_k * len(lens_k)
+    need = runner.splitkv_paged_workspace_size(len(lens_k), h, kvh, max_q, max_k, len(q), total, ps, table.shape[1],
+                                               first, splits, causal=causal)
+    ws = torch.empty(need, device=dev, dtype=torch.uint8)
+    return lambda: runner.call_splitkv_paged(q, kc, vc, o, None, cu_q, keys, table, max_q, max_k, splits,
+                                             workspace=ws, total_k=sum(lens_k) if total_k else None, causal=causal)
+
+
+def test_short_sequences_beside_a_long_one(gpu_runner):
+    """Decode: 63 sequences of 50 keys beside one of 200000 (H32 KVH8) cost a
+    few percent of the long one (165 us against 155), not what a workgroup
+    takes for 50 of them in a row (352 us)."""
+    import torch
+    print("  decode 63 x 50 keys + 200000", flush=True)
+    both = _paged(torch, gpu_runner, 32, 8, [1] * 64, [50] * 63 + [200000])
+    alone = _paged(torch, gpu_runner, 32, 8, [1], [200000])
+    assert _ratio(torch, both, alone) < 1.6
