@@ -60,3 +60,18 @@ def test_short_sequences_beside_a_long_one(gpu_runner):
     both = _paged(torch, gpu_runner, 32, 8, [1] * 64, [50] * 63 + [200000])
     alone = _paged(torch, gpu_runner, 32, 8, [1], [200000])
     assert _ratio(torch, both, alone) < 1.6
+
+
+def test_ragged_decode_of_several_q_tiles(gpu_runner):
+    """Decode of 16 queries of 8 heads on one K/V head (four 32-row tiles, 41
+    sequences of 24000-30000 keys): Auto's equal ranges are no slower than the
+    chunks of its plan (the tiles of a range share its keys in one XCD's L2;
+    spread over the XCDs they read them four times)."""
+    import torch
+    lens = [24000 + 157 * i for i in range(41)]
+    print("  decode 41 x 16 queries H8 KVH1", flush=True)
+    auto = _paged(torch, gpu_runner, 8, 1, [16] * 41, lens, causal=2)
+    plan = gpu_runner.splitkv_paged_select(41, 8, 1, 16, max(lens), 41 * 16, sum(lens), 64, -(-max(lens) // 64),
+                                           sum(-(-n // 64) for n in lens), causal=2)
+    chunks = _paged(torch, gpu_runner, 8, 1, [16] * 41, lens, causal=2, splits=plan)
+    assert _ratio(torch, auto, chunks) < 1.15
