@@ -395,7 +395,8 @@ class Runner:
         """q/o: [total_q, heads, 128]; k_cache/v_cache: [num_pages, page_size, kv_heads, 128] (BF16,
         contiguous); cu_q: int32 [batch+1]; seqlens_k: int32 [batch]; block_table: int32
         [batch, max_pages_per_seq] (device tensors); lse: FP32 [heads, total_q] or None.  total_k
-        (cached keys over the batch) only steers Auto; None passes max_k * batch."""
+        (cached keys over the batch) only steers Auto: max_k * batch says that every sequence has
+        max_k keys; None (not known) passes one less than that for two sequences or more."""
         import torch
         assert all(x.dtype == torch.bfloat16 and x.is_cuda and x.is_contiguous() for x in (q, k_cache, v_cache, o))
         assert q.dim() == 3 and q.shape[2] == D and o.shape == q.shape
@@ -405,10 +406,12 @@ class Runner:
         tq, h, _ = q.shape
         assert lse is None or (tuple(lse.shape) == (h, tq) and lse.is_contiguous() and lse.dtype == torch.float32)
         b = seqlens_k.numel()
+        if total_k is None:
+            total_k = int(max_k) * b - (b > 1)
         return PagedArgs(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), o.data_ptr(),
                          lse.data_ptr() if lse is not None else None, cu_q.data_ptr(), seqlens_k.data_ptr(),
                          block_table.data_ptr(), b, h, k_cache.shape[2], int(max_q), int(max_k), tq,
-                         int(max_k) * b if total_k is None else int(total_k), k_cache.shape[0], k_cache.shape[1],
+                         int(total_k), k_cache.shape[0], k_cache.shape[1],
                          block_table.shape[1], 1 / math.sqrt(D) if scale is None else scale)
 
     @staticmethod

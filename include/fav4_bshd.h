@@ -250,6 +250,9 @@ struct Fav4PagedArgs {
 // [0, max_seqlen_k], page numbers to [0, num_pages)), so malformed tables give
 // undefined results but no access outside the buffers.  A sequence with no
 // keys gets O = 0 and LSE = -inf; one with no queries writes nothing.
+//  * total_k = batch * max_seqlen_k says that every sequence has max_seqlen_k
+//    keys; a caller that does not know the sum passes one less (the plan is
+//    the same), and Auto decode then goes by the lengths on the device.
 //  * splits: 0 = the Auto count of fav4_bshd_forward_splitkv_varlen on these
 //    sizes, else 1..256; either is raised if needed so that no chunk of the plan
 //    spans more than 64 key tiles.  One chunk still runs the split kernels.

@@ -795,3 +795,20 @@ def test_bottom_right_prefill_plans(lib, shape):
     pages = -(-s_ // 64)
     assert runner.splitkv_paged_select(b, h, h, s_, s_, b * s_, b * s_, 64, pages, b * pages, causal=2) == \
         -(-ktiles // min(tps_p, 64))
+
+
+@pytest.mark.parametrize("shape", [(2, 8, 8, 1, 1), (2, 32, 8, 1, 30000), (105, 12, 3, 1, 2545), (256, 8, 1, 16, 33),
+                                   (7, 4, 4, 700, 9001), (300, 8, 2, 4, 500000)])
+def test_paged_unknown_total_keeps_the_plan(lib, shape):
+    """One key less than batch * max_seqlen_k (what Runner passes for an unknown
+    total) gives the plan and the workspace of the full total."""
+    b, h, kvh, mq, mk = shape
+    ps = 64
+    got = []
+    for total in (b * mk, b * mk - 1):
+        a = _pgood(batch=b, heads=h, kv_heads=kvh, max_seqlen_q=mq, max_seqlen_k=mk, total_k=total, total_q=b * mq,
+                   page_size=ps, max_pages_per_seq=-(-mk // ps), q=None, k_cache=None, v_cache=None, o=None,
+                   cu_seqlens_q=None, seqlens_k=None, block_table=None)
+        got.append([(lib.fav4_bshd_splitkv_paged_select(C.byref(a), causal),
+                     lib.fav4_bshd_splitkv_paged_workspace_size(C.byref(a), causal, 0)) for causal in (0, 2)])
+    assert got[0] == got[1] and min(x for pair in got[0] for x in pair) > 0

@@ -75,3 +75,14 @@ def test_ragged_decode_of_several_q_tiles(gpu_runner):
                                            sum(-(-n // 64) for n in lens), causal=2)
     chunks = _paged(torch, gpu_runner, 8, 1, [16] * 41, lens, causal=2, splits=plan)
     assert _ratio(torch, auto, chunks) < 1.15
+
+
+def test_ragged_decode_without_a_total(gpu_runner):
+    """Decode of 105 sequences of 324-2545 keys (H12 KVH3) when the caller does
+    not say how many keys there are: no slower than when it does."""
+    import torch
+    lens = np.random.default_rng(3).integers(324, 2546, size=105).tolist()
+    print("  decode 105 ragged, no total", flush=True)
+    unknown = _paged(torch, gpu_runner, 12, 3, [1] * 105, lens, total_k=False)
+    known = _paged(torch, gpu_runner, 12, 3, [1] * 105, lens)
+    assert _ratio(torch, unknown, known) < 1.12
