@@ -118,10 +118,10 @@ constexpr int MIN_TILES_PER_SPLIT = 4;   // Auto keeps >= 4 key tiles per chunk
 constexpr int MAX_SPLIT_SQ = 1 << 22;    // keeps a chunk's O rows under a 4 GiB buffer bound
 constexpr int DECODE_SQ = 32;            // up to this many queries: the one-wave decode shape
 
-// Tile shape of the partial kernel: 8 waves x 256-row q tiles x 64-key tiles
-// (one workgroup fills a CU), 4 waves x 128 rows (two per CU) where 256 rows
-// would leave half the waves without a query, or for decode 1 wave x 32 rows x
-// 32-key tiles (three workgroups per CU, each with 48 KiB of LDS).
+// Tile shape that a plan assumes: 8 waves x 256-row q tiles x 64-key tiles (one
+// workgroup fills a CU), or for decode 1 wave x 32 rows x 32-key tiles (three
+// workgroups per CU, each with 48 KiB of LDS).  Packed and paged prefill may
+// run 128-row tiles instead (packed_prefill_run).
 struct SplitShape {
     int bm, bn, wgs_per_cu, auto_max;
 };
@@ -344,8 +344,12 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
             if (VARLEN && a.batch <= fav4::MAX_SORTED_SEQS)
                 total = std::min(total, a.heads * p.splits *
                                             ((sp.total_q + int64_t(a.batch) * (p.shape.bm - 1)) / p.shape.bm));
-            if (p.shape.bm == 128) launch_chunks<CAUSAL, KV, BR, 4>(a, kv_heads, p, sp, total, stream);
-            else launch_chunks<CAUSAL, KV, BR, 8, KV == 0 ? 3 : 2>(a, kv_heads, p, sp, total, stream);
+            if constexpr (KV == 0) {
+                launch_chunks<CAUSAL, KV, BR, 8, 3>(a, kv_heads, p, sp, total, stream);
+            } else {
+                if (p.shape.bm == 128) launch_chunks<CAUSAL, KV, BR, 4>(a, kv_heads, p, sp, total, stream);
+                else launch_chunks<CAUSAL, KV, BR, 8>(a, kv_heads, p, sp, total, stream);
+            }
         }
     } else if (VARLEN && p.ranges > 0) {
         if constexpr (VARLEN) {

@@ -29,3 +29,10 @@ def test_merge_keeps_its_waves(resources, per):
     for name, r in kernels.items():
         assert r["Occupancy [waves/SIMD]"] >= MERGE_WAVES[per], (name, r)
         assert r["ScratchSize [bytes/lane]"] == 0, name
+
+
+def test_contiguous_prefill_chunks_have_one_shape(resources):
+    """Split-KV plans of contiguous K/V have 256-row q tiles only: the 128-row
+    chunk kernel is built for packed and paged K/V alone."""
+    rows128 = [n for n in resources if re.search(r"fwd_kernel_chunkILb[01]ELb[01]ELi4E", n)]
+    assert rows128 and not [n for n in rows128 if "Li4ELi0E" in n]
