@@ -299,6 +299,18 @@ int split_args_ok(const Fav4Args* a, int kv_heads, int causal, int splits) {
     return st != hipSuccess ? st : split_shape_ok(a, kv_heads, causal, splits);
 }
 
+// Packed and paged prefill on 256-row tiles keeps two key tiles in flight
+// (three LDS stages) where at most half of its waves have queries and a chunk is
+// long enough to pay for the two tiles it prefetches in vain: it then waits for
+// K/V.  One and two tiles in flight, K/V from memory (several caches in turn):
+// 2 x 40 queries H8, chunks of 24 tiles 44.9 and 38.0 us, of 16 33.7 and 29.7;
+// 4 x 80 H8, of 31 66.2 and 61.4, of 12 34.7 and 33.5, of 8 27.4 and 27.1; 64 x
+// 64 H4, of 16 35.0 and 31.8.  With K/V in the memory-side cache they are even
+// from 16 tiles on, and 5% apart the other way below 8.  4 x 1024 queries on
+// 4096 keys H32 lose 3% by it.
+constexpr int STREAM_SQ = 128;
+constexpr int STREAM_TPS = 12;
+
 // Prefill chunks: K/V in BSHD (KV 0), packed (1) or paged (2) layout.
 template <bool CAUSAL, int KV, bool BR, int WAVES, int STAGES = 2>
 void launch_chunks(const Fav4Args& a, int kv_heads, const SplitPlan& p, const fav4::SplitArgs& sp, int64_t total,
@@ -348,6 +360,8 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
                 launch_chunks<CAUSAL, KV, BR, 8, 3>(a, kv_heads, p, sp, total, stream);
             } else {
                 if (p.shape.bm == 128) launch_chunks<CAUSAL, KV, BR, 4>(a, kv_heads, p, sp, total, stream);
+                else if (a.sq <= STREAM_SQ && p.tps >= STREAM_TPS)
+                    launch_chunks<CAUSAL, KV, BR, 8, 3>(a, kv_heads, p, sp, total, stream);
                 else launch_chunks<CAUSAL, KV, BR, 8>(a, kv_heads, p, sp, total, stream);
             }
         }

@@ -1355,9 +1355,9 @@ __device__ __forceinline__ int visible_keys(int mask, int q0, int bm, int sq, in
 // chunk gives; the others write their partials row-contiguously for
 // combine_kernel.
 // STAGES: BSHD calls, whose few q tiles mostly stream K/V, keep three LDS
-// stages (prefetch distance 2; B2 H16 128 x 65536 200 us, 212 with two); packed
-// and paged ones, which fill the GPU, run two (4 x 1024 x 4096 H32 205 us, 211
-// with three).
+// stages (prefetch distance 2; B2 H16 128 x 65536 200 us, 212 with two), as do
+// packed and paged calls of few queries; the other packed and paged ones run
+// two (4 x 1024 x 4096 H32 205 us, 211 with three).
 // KV: where K/V lie.  0: BSHD, 1: packed sequences, 2: paged caches.  Packed
 // and paged items come from the sequences' lengths (sorted_item), heaviest
 // chunks first, so that a sequence with few keys or queries costs what it has:

@@ -285,6 +285,23 @@ def _check_bottom_right(o, lse, q, k, v, cu_q, cu_k, lens, group, splits):
             assert orc.check_acceptance_tolerance(e) and orc.check_reference_tolerance(e), (splits, i, e)
 
 
+def _check_dense(o, lse, q, k, v, cu_q, cu_k, lens, group):
+    """Every sequence of a dense output against the FP64 oracle."""
+    for i, (sq, sk) in enumerate(lens):
+        a, b = cu_q[i], cu_q[i + 1]
+        c, d = cu_k[i], cu_k[i + 1]
+        if sq == 0:
+            continue
+        got, got_lse = to_host_bits(o[a:b])[None], lse[:, a:b].cpu().numpy()[None]
+        if sk == 0:
+            assert (orc.bf16_to_f32(got) == 0).all() and (got_lse == -np.inf).all(), i
+            continue
+        ke, ve = (np.repeat(x[c:d][None], group, axis=2) for x in (k, v))
+        ref, ref_lse = orc.attention_fp64(q[a:b][None], ke, ve, orc.DEFAULT_SCALE, False)
+        e = orc.errors(got, got_lse, ref, ref_lse)
+        assert orc.check_acceptance_tolerance(e) and orc.check_reference_tolerance(e), (i, sq, sk, e)
+
+
 @pytest.mark.parametrize("ps", [64, 256])
 def test_splitkv_paged_prefill(gpu_runner, ps):
     """Queries longer than 32 over paged caches (the 8-wave shape): dense and
@@ -432,6 +449,54 @@ def test_paged_prefill_chunks(gpu_runner, case):
         seen = torch.isfinite(whole_lse)
         assert torch.equal(torch.isfinite(lse), seen) and torch.equal(torch.isfinite(lse3), seen)
         assert (lse[seen] - whole_lse[seen]).abs().max().item() <= 2e-4, splits
+
+
+# (heads, kv_heads, page_size, [(sq, sk), ...], splits): chunks of 12 key tiles
+# and more under at most 128 queries (three LDS stages; 11 tiles and 129 queries
+# have two), with chunks of one and two tiles, queries without keys, keys without
+# queries, and more pages than a wave's lanes.
+FEW_QUERY_CASES = [
+    (2, 1, 64, [(33, 5000), (128, 4097), (1, 768), (100, 0), (0, 300), (40, 30), (7, 65)], 6),
+    (3, 3, 64, [(128, 64 * 24), (127, 64 * 24 - 63), (90, 64 * 12), (64, 64 * 12 + 1)], 2),
+    (3, 3, 64, [(128, 64 * 22), (33, 64 * 11 + 1)], 2),
+    (3, 3, 64, [(129, 64 * 24), (33, 64 * 12 + 1)], 2),
+    (1, 1, 64, [(97, 9000), (34, 700)], 1),
+    (2, 2, 128, [(61, 6001), (128, 3333), (90, 90)], 0),
+]
+
+
+@pytest.mark.parametrize("case", FEW_QUERY_CASES, ids=lambda c: "h%dkv%d_p%d_n%d_s%d" % (*c[:3], len(c[3]), c[4]))
+def test_prefill_of_few_queries(gpu_runner, case):
+    """Paged prefill, dense and bottom-right, and packed bottom-right, against
+    the FP64 oracle, on a workspace full of NaN; nothing is written past O, LSE
+    and the workspace."""
+    import torch
+    h, kvh, ps, lens, splits = case
+    q, k, v, kc, vc, cu_q, cu_k, seqlens_k, table = _build(h, kvh, ps, lens, seed=211)
+    dev = torch.device("cuda:0")
+    group = h // kvh
+    qd, kd, vd, kcd, vcd = (to_device(x, dev) for x in (q, k, v, kc, vc))
+    cq, ck, sk_d, tb = (torch.from_numpy(x).to(dev) for x in (cu_q, cu_k, seqlens_k, table))
+    max_q, max_k, tq = max(s for s, _ in lens), max(s for _, s in lens), len(q)
+    sizes = (len(lens), h, kvh, max_q, max_k, tq, len(k))
+    for paged, causal in ((True, 0), (True, 2), (False, 2)):
+        print(f"  few queries h{h} kv{kvh} n{len(lens)} splits {splits} paged {paged} causal {causal}", flush=True)
+        need = gpu_runner.splitkv_paged_workspace_size(*sizes, ps, table.shape[1], len(kc), splits, causal=causal) \
+            if paged else gpu_runner.splitkv_varlen_workspace_size(*sizes, causal, splits)
+        ws = torch.full((need // 4 + GUARD,), float("nan"), device=dev, dtype=torch.float32)
+        ob, lb, o, lse = _out(torch, dev, tq, h, True)
+        if paged:
+            gpu_runner.call_splitkv_paged(qd, kcd, vcd, o, lse, cq, sk_d, tb, max_q, max_k, splits, workspace=ws,
+                                          total_k=len(k), causal=causal)
+        else:
+            gpu_runner.call_splitkv_varlen(qd, kd, vd, o, lse, cq, ck, max_q, max_k, causal, splits, workspace=ws)
+        torch.cuda.synchronize()
+        for guard in (ob[tq:], lb[h * tq:], ws[need // 4:]):
+            assert torch.isnan(guard).all().item(), (paged, causal)
+        if causal == 2:
+            _check_bottom_right(o, lse, q, k, v, cu_q, cu_k, lens, group, splits)
+        else:
+            _check_dense(o, lse, q, k, v, cu_q, cu_k, lens, group)
 
 
 # (heads, kv_heads, page_size, [(sq, sk), ...], causal): ragged decode batches
