@@ -551,16 +551,28 @@ SplitPlan packed_decode_run(const Fav4Args& a, int kv_heads, int64_t total_k, co
 // runs: the q tile (128 or 256 rows) and, for Auto, the chunk count up to the
 // plan's (which sizes the workspace) with the lowest predicted time.  The
 // plan takes every sequence as long as the longest; this model takes the
-// batch's means as well (microseconds, graph-timed on MI355X; a chunk costs
-// 9-10 plus c per key tile; a merged row's chunks are written and read once
-// more):
-//  * lengths near the longest (mean >= 3/4): whole rounds of equal chunks;
-//  * else the average load per resident workgroup plus a tenth of the longest
-//    item, or that item (the lists start the long items first).
-// On eight batches (1-8 sequences of 86-2048 queries against 1k-32k keys, H16
-// and H32) over 1-16 chunks and both tiles it picks the fastest measured choice
-// or one within 9% of it.  Merging costs what a second pass over FP32 partials
-// does: 4 x 1024 queries against 4096 keys H32 217 us in one chunk, 290 in two.
+// batch's means as well (microseconds; fitted to 1558 graph-timed runs on MI355X:
+// 255 random batches of 1-64 sequences, 33-2048 queries, 64-60000 keys, H1-128,
+// over up to 11 chunk counts and both tiles).  A chunk costs 7 plus c per key
+// tile: 128-row tiles c = 1.1 with at most one workgroup per CU, 1.5 with two;
+// 256-row ones 1.0 where half of their waves have no query, else 1.45.
+//  * Chunks that are resident at once take one chunk's time (10% more where
+//    some CUs have two).
+//  * Lengths near the longest (mean >= 3/4): whole rounds of equal chunks; from
+//    the third on their ends spread and half a round is left over.
+//  * Other lengths: the average load per resident workgroup and half a chunk
+//    (the lists start the long chunks first), and never less than the longest.
+//  * Merging writes and reads FP32 partials: 4 x 1024 queries against 4096 keys
+//    H32 217 us in one chunk, 290 in two.
+// Other counts than the plan's must promise 4%, and are not taken where the
+// caller does not know the key total (one less than the most), since the lengths
+// may be anything: 43 of 24..94 queries on 6630..52830 keys H4 640 us in the
+// chunks that equal lengths would want, 556 in the plan's 13.  On 245 other
+// batches the choice is 1.5% behind the fastest of the runs on average (at a
+// given chunk count 0.8%), and 7 are slower by more than 2% than the 256-row
+// chunks of the plan's count that every batch once had, the worst by 17% (1.56x
+// on average).  With 9 + 1.1 or 10 + 1.75 per tile and half a q tile counted for
+// a sequence with fewer queries than one, it was 4.2% behind, the worst 1.8x.
 SplitPlan packed_prefill_run(const Fav4Args& a, int64_t total_q, int64_t total_k, bool br, const SplitPlan& p,
                              bool choose) {
     const int ktiles = (a.sk + 63) / 64;
@@ -570,27 +582,32 @@ SplitPlan packed_prefill_run(const Fav4Args& a, int64_t total_q, int64_t total_k
     const bool uniform = 4 * mean_k >= 3.0 * a.sk;
     const double mean = std::max(1.0, mean_k / 64 + 0.5 - (br ? 0.5 * mean_q / 64 : 0.0));   // key tiles per q tile
     auto predict = [&](int bm, int splits, int tps) {
-        const double slots = bm == 256 ? cus : 2 * cus;
-        const double qtiles = a.heads * std::min(seqs * ((a.sq + bm - 1) / bm), double(total_q) / bm + 0.5 * seqs);
-        const double chunks = std::max(1.0, std::ceil(mean / tps - 0.25)), items = qtiles * chunks;
-        const double fixed = bm == 256 ? 9.0 : 10.0;
-        const double per_tile = bm == 256 ? (a.sq > 128 ? 1.7 : 1.1) : (items > cus ? 1.75 : 1.1);
+        const double slots = bm == 256 ? cus : 2 * cus, fixed = 7.0;
+        const double qtiles = a.heads * seqs * std::min<double>((a.sq + bm - 1) / bm, std::max(1.0, mean_q / bm + 0.5));
+        const double chunks = std::max(1.0, uniform ? std::ceil(mean / tps - 0.25) : mean / tps + 0.4);
+        const double items = qtiles * chunks, rounds = items / slots;
+        const double alone = bm == 128 ? 1.1 : a.sq <= 128 ? 1.0 : 1.45;       // per key tile, one workgroup on the CU
+        const bool shared = bm == 128 && items > cus;
+        const double per_tile = shared ? 1.5 : alone, longest = fixed + alone * std::min(tps, ktiles);
+        const double chunk = fixed + per_tile * std::min<double>(tps, mean);
         double t;
-        if (uniform) {
-            t = std::ceil(items / slots) * (fixed + per_tile * std::min<double>(tps, mean));
-        } else {
-            const double longest = fixed + std::min(per_tile, bm == 256 ? 1.6 : 1.4) * tps;
-            t = std::max(longest, qtiles * (chunks * fixed + per_tile * mean) / slots + 0.1 * longest);
-        }
+        if (rounds <= 1)
+            t = fixed + (chunk - fixed) * (shared ? 1.1 : 1.0);
+        else if (uniform)
+            t = chunk * (rounds <= 2.02 ? 2.0 : rounds + 0.5);
+        else
+            t = qtiles * (chunks * fixed + per_tile * mean) / slots + 0.5 * (fixed + per_tile * std::min(tps, ktiles));
+        t = std::max(t, longest);
         if (splits > 1)
-            t += 5.0 + double(total_q) * a.heads * splits * 1040 / 4.5e6 *
-                           (uniform ? 1.0 : std::max(0.3, mean_k / a.sk));
-        return t;
+            t += 3.5 + double(total_q) * a.heads * splits * 1040 / 3e6 * (uniform ? 1.0 : std::max(0.3, mean_k / a.sk));
+        return tps == p.tps ? t : 1.04 * t;
     };
+    const bool unknown = a.batch > 1 && total_k == int64_t(a.batch) * a.sk - 1;
+    const int fewest = choose && !unknown ? 1 : p.splits;
     SplitPlan best = p;
     double best_t = 0;
     bool first = true;
-    for (int s = choose ? 1 : p.splits; s <= p.splits; ++s) {
+    for (int s = fewest; s <= p.splits; ++s) {
         const int tps = s == p.splits ? p.tps : (ktiles + s - 1) / s, splits = (ktiles + tps - 1) / tps;
         for (int bm : {256, 128}) {
             const double t = predict(bm, splits, tps);

@@ -107,3 +107,27 @@ def test_paged_prefill_of_few_queries(gpu_runner):
                                                                                    workspace=ws))
     all_of = lambda calls: lambda: [c() for c in calls]
     assert _ratio(torch, all_of(paged), all_of(contiguous), calls=3) < 1.18
+
+
+# (heads, kv_heads, causal, total known, [(sq, sk), ...]) where a count that
+# looked cheap was not: one query tile of every sequence counted as half a one;
+# unknown lengths; the last q tile of a square bottom-right batch.
+PREFILL = {
+    "short_queries": (32, 8, 0, True, [(40 + 2 * i, 22000 + 300 * i) for i in range(11)]),
+    "unknown_total": (4, 4, 2, False, [(24 + 5 * (i % 14), 6630 + 1100 * i) for i in range(43)]),
+    "square": (8, 8, 2, True, [(4096, 4096)]),
+}
+
+
+@pytest.mark.parametrize("name", PREFILL)
+def test_prefill_auto_against_its_plan(gpu_runner, name):
+    """Auto prefill over paged caches is no slower than its plan's chunk count."""
+    import torch
+    h, kvh, causal, known, lens = PREFILL[name]
+    lq, lk = [s for s, _ in lens], [s for _, s in lens]
+    print(f"  paged prefill {name}", flush=True)
+    auto = _paged(torch, gpu_runner, h, kvh, lq, lk, causal=causal, total_k=known)
+    plan = gpu_runner.splitkv_paged_select(len(lens), h, kvh, max(lq), max(lk), sum(lq), sum(lk), 64,
+                                           -(-max(lk) // 64), sum(-(-n // 64) for n in lk), causal=causal)
+    chunks = _paged(torch, gpu_runner, h, kvh, lq, lk, causal=causal, splits=plan)
+    assert _ratio(torch, auto, chunks) < 1.08
