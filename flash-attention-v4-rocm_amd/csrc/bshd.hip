@@ -419,10 +419,8 @@ constexpr int BOTTOM_RIGHT = 2;
 constexpr int BY_ITEM_ROUNDS = 4;
 
 template <int WAVES>
-void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int total, hipStream_t stream) {
+void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int total, int key_bits, hipStream_t stream) {
     const dim3 grid = item_grid(total), block(WAVES * 64);
-    int key_bits = 1;                          // of the longest sequence's key tile count
-    while (((a.max_seqlen_k + 63) / 64) >> key_bits) ++key_bits;
     const int slots = device_cus() * 8 / WAVES;            // workgroups resident at once
     const bool by_item = total <= BY_ITEM_ROUNDS * slots;
     if (causal == BOTTOM_RIGHT && a.lse)
@@ -798,14 +796,26 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_varlen(c
     const int tiles = (a->max_seqlen_q + bm - 1) / bm;
     int64_t total = int64_t(a->batch) * a->heads * tiles;
     if (total > INT_MAX) return hipErrorInvalidValue;
-    // The sorted item lists hold only the q tiles that exist, and no batch of
-    // total_q rows has more than this many of them.
-    if (a->batch <= fav4::MAX_SORTED_SEQS)
+    // The sorted item lists' key_bits: the bits of the key tiles that a q tile
+    // can see; 0 means no lists.  Batches of one q tile and one key tile a
+    // sequence have nothing to sort, and the search would cost their short items
+    // 4-10% (sorted and not: H32 KVH8 256 x 16 tokens 73.4 and 68.9 us, 211 of
+    // 5..41 causal on up to 1934 keys 76.6 and 69.0).  Two key tiles go either
+    // way: H16 KVH8 43 of 56..72 tokens 13.7 and 15.2, H10 KVH5 165 of 12..98
+    // causal on up to 2028 keys 28.4 and 26.4.
+    const int keys = causal == 1 ? std::min(a->max_seqlen_q, a->max_seqlen_k) : a->max_seqlen_k;
+    const int key_tiles = (keys + 63) / 64;
+    int key_bits = 0;
+    if (a->batch <= fav4::MAX_SORTED_SEQS && (tiles > 1 || key_tiles > 1)) {
+        while (key_tiles >> key_bits) ++key_bits;
+        // The lists hold only the q tiles that exist, and no batch of total_q
+        // rows has more than this many of them.
         total = std::min(total, a->heads * ((a->total_q + int64_t(a->batch) * (bm - 1)) / bm));
+    }
     if (small)
-        launch_varlen<4>(*a, causal, tiles, int(total), stream);
+        launch_varlen<4>(*a, causal, tiles, int(total), key_bits, stream);
     else
-        launch_varlen<8>(*a, causal, tiles, int(total), stream);
+        launch_varlen<8>(*a, causal, tiles, int(total), key_bits, stream);
     return hipGetLastError();
 }
 

@@ -1614,23 +1614,23 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
         const int ke = min(max(a.cu_seqlens_k[b + 1], ks), min(a.total_k, ks + a.max_seqlen_k));
         return Span{qs, qe, ks, ke};
     };
-    // Item order, up to MAX_SORTED_SEQS sequences: sorted_item's lists.  A q
+    // Item order, with key_bits (up to MAX_SORTED_SEQS sequences, unless there is
+    // nothing to sort): sorted_item's lists.  A q
     // tile weighs its key tiles (by_item: with few items per workgroup slot,
     // where the last ones decide) or its sequence's longest tile's (its q
     // tiles then run together, heaviest first, and share its K/V in L2).
-    // Larger batches: column_item, within a pair the q tiles last-to-first.
+    // Else: column_item, within a pair the q tiles last-to-first.
     // The lists against that order (graph-timed, causal): 24 sequences of 64..4096
     // tokens H32 KVH8 708 -> 582 us, 64 of 100..1000 H8 69 -> 55, 4 x 2048
     // H16 105 -> 77 (by sequence 97), 8 x 4096 H8 313 -> 264 (313); 32 of
     // 1024..7168 H8 858 -> 848.
-    const bool sorted = a.batch <= MAX_SORTED_SEQS;
     {
         const uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;
         if (wg >= uint32_t(total)) return;
         const int id = int(wg);
         int batch, head, tile;
         Span sp;
-        if (sorted) {
+        if (key_bits > 0) {
             int rank;
             packed_head_rank(id, a.heads, head, rank);
             const PackedItem it = sorted_item<BM, BN>(rank, a.batch, key_bits, lane, [&](int b) {

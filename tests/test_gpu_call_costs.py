@@ -131,3 +131,18 @@ def test_prefill_auto_against_its_plan(gpu_runner, name):
                                            -(-max(lk) // 64), sum(-(-n // 64) for n in lk), causal=causal)
     chunks = _paged(torch, gpu_runner, h, kvh, lq, lk, causal=causal, splits=plan)
     assert _ratio(torch, auto, chunks) < 1.08
+
+
+def test_short_packed_sequences(gpu_runner):
+    """256 packed sequences of 16 tokens (H32 KVH8) take no longer than 257,
+    which are too many for sorted item lists: there is nothing to sort."""
+    import torch
+    print("  packed 256 x 16 and 257 x 16", flush=True)
+    calls = []
+    for n in (256, 257):
+        mk = lambda heads: torch.randn((n * 16, heads, 128), device="cuda").to(torch.bfloat16)
+        q, k, v = mk(32), mk(8), mk(8)
+        o = torch.empty_like(q)
+        cu = torch.arange(n + 1, device="cuda", dtype=torch.int32) * 16
+        calls.append(lambda q=q, k=k, v=v, o=o, cu=cu: gpu_runner.call_varlen(q, k, v, o, None, cu, cu, 16, 16, False))
+    assert _ratio(torch, *calls, calls=50) < 1.035

@@ -209,9 +209,11 @@ def test_varlen_bottom_right_causal(gpu_runner, case):
 
 # (heads, kv_heads, sequences, longest): batches at the edges of the item
 # lists (one, and either side of 64 and of 256 sequences), heads in whole
-# XCD shares and not, few items per workgroup slot and many, both tile sizes.
+# XCD shares and not, few items per workgroup slot and many, both tile sizes;
+# the last four: short sequences on both sides of what is sorted at all, most
+# of them without a query in one.
 LIST_CASES = [(1, 1, 1, 300), (3, 1, 63, 300), (8, 8, 64, 130), (16, 2, 65, 700), (8, 2, 255, 260), (16, 4, 256, 300),
-              (5, 5, 257, 200), (32, 4, 40, 1300)]
+              (5, 5, 257, 200), (32, 4, 40, 1300), (3, 3, 256, 64), (8, 2, 70, 64), (8, 2, 70, 65), (4, 4, 200, -60)]
 
 
 @pytest.mark.parametrize("case", LIST_CASES, ids=lambda c: "h%dkv%d_n%d_max%d" % c)
@@ -222,7 +224,10 @@ def test_varlen_item_lists(gpu_runner, case):
     import torch
     h, kvh, n, longest = case
     rng = np.random.default_rng(n * 1000 + h)
+    sparse, longest = longest < 0, abs(longest)
     sq = rng.integers(0, longest + 1, n)
+    if sparse:
+        sq[rng.random(n) < 0.95] = 0
     sk = rng.integers(0, longest + 1, n)
     edges = np.array([0, 1, 127, 128, 129, 255, 256, 257, longest])
     sq[:edges.size] = np.minimum(edges, longest)[:n]
