@@ -410,19 +410,22 @@ int launch_split(const Fav4Args& a, int kv_heads, const SplitPlan& p, void* ws, 
 // with sq queries and sk keys sees keys j <= sk - sq + i).
 constexpr int BOTTOM_RIGHT = 2;
 
-// Up to this many items per resident workgroup, the packed kernel's lists go
-// by each q tile's own keys, else by its sequence's: with few rounds the last
-// items decide (4 x 2048 tokens H16 causal, 1 round: 77 us by tile, 97 by
+// Up to this many items per resident workgroup (rounds), a causal packed batch's
+// lists go by each q tile's own keys, else by its sequence's: with few rounds the
+// last items decide (4 x 2048 tokens H16, 2 rounds: 77 us by tile, 97 by
 // sequence; 8 x 4096 H8, 4 rounds: 264 and 313), with many the q tiles of a
-// sequence profit from running together (32 x 1024..7168 H8, 8 rounds: 874 and
-// 844; 8 x 4096 H32, 16 rounds: 1092 and 1065).
-constexpr int BY_ITEM_ROUNDS = 4;
+// sequence profit from running together (32 x 1024..7168 H8, 16 rounds: 874 and
+// 844; 8 x 4096 H32, 16 rounds: 1092 and 1065), the earlier the fewer they are.
+// By sequence over by tile, means of 330 random batches: 2 or 3 q tiles, 2-4
+// rounds 0.94 (0.87 at worst), up to 2 rounds 1.02; 4-7 tiles, 3-4 rounds 0.88,
+// 2-3 rounds 1.10; 8 or more, 3-4 rounds 1.09.
+int by_item_rounds(int tiles) { return tiles < 4 ? 2 : tiles < 8 ? 3 : 4; }
 
 template <int WAVES>
 void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int total, int key_bits, hipStream_t stream) {
     const dim3 grid = item_grid(total), block(WAVES * 64);
     const int slots = device_cus() * 8 / WAVES;            // workgroups resident at once
-    const bool by_item = total <= BY_ITEM_ROUNDS * slots;
+    const bool by_item = total <= by_item_rounds(tiles) * slots;
     if (causal == BOTTOM_RIGHT && a.lse)
         hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, true, WAVES, true>), grid, block, 0, stream, a,
                            tiles, total, key_bits, by_item);
