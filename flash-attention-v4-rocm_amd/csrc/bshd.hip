@@ -421,29 +421,48 @@ constexpr int BOTTOM_RIGHT = 2;
 // 2-3 rounds 1.10; 8 or more, 3-4 rounds 1.09.
 int by_item_rounds(int tiles) { return tiles < 4 ? 2 : tiles < 8 ? 3 : 4; }
 
+// The grid of a packed call's lists of n items a head (packed_head_rank's ids).
+int64_t list_ids(int64_t n, int heads, int block_bits) {
+    if ((heads & 7) == 0) return n * heads;
+    const int64_t blocks = heads * ((n + (int64_t(1) << block_bits) - 1) >> block_bits);
+    return ((blocks + 7) / 8 * 8) << block_bits;
+}
+
 template <int WAVES>
-void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int total, int key_bits, hipStream_t stream) {
-    const dim3 grid = item_grid(total), block(WAVES * 64);
+void launch_varlen(const Fav4VarlenArgs& a, int causal, int tiles, int64_t items, int key_bits, hipStream_t stream) {
     const int slots = device_cus() * 8 / WAVES;            // workgroups resident at once
-    const bool by_item = total <= by_item_rounds(tiles) * slots;
+    const bool by_item = causal && items <= int64_t(by_item_rounds(tiles)) * slots;
+    // By sequence, sequences of up to 4 q tiles: the ranks go to the XCDs in blocks
+    // of that many, so that a sequence's tiles share its K/V in one L2 and a short
+    // last tile is not always the same XCD's (56 x 148 tokens dense H4 15.8 and
+    // 12.4 us); with 16 blocks an XCD or more, to keep the XCDs even, and none
+    // that would make one round two.  Longer ones: rank by rank (4 x 4096 causal
+    // H20, 5 rounds, in blocks of 8 372 us, else 333).  -1: by tile.
+    int block_bits = by_item ? -1 : 0;
+    if (!by_item && tiles <= 4) {
+        while ((1 << block_bits) < tiles) ++block_bits;
+        if (items >> block_bits < 128 || (items <= slots && items + (8 << block_bits) > slots)) block_bits = 0;
+    }
+    const int total = int(key_bits ? list_ids(items / a.heads, a.heads, std::max(0, block_bits)) : items);
+    const dim3 grid = item_grid(total), block(WAVES * 64);
     if (causal == BOTTOM_RIGHT && a.lse)
         hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, true, WAVES, true>), grid, block, 0, stream, a,
-                           tiles, total, key_bits, by_item);
+                           tiles, total, key_bits, block_bits);
     else if (causal == BOTTOM_RIGHT)
         hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, false, WAVES, true>), grid, block, 0, stream, a,
-                           tiles, total, key_bits, by_item);
+                           tiles, total, key_bits, block_bits);
     else if (causal && a.lse)
         hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, true, WAVES>), grid, block, 0, stream, a, tiles, total,
-                           key_bits, by_item);
+                           key_bits, block_bits);
     else if (causal)
         hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, true, false, WAVES>), grid, block, 0, stream, a, tiles, total,
-                           key_bits, by_item);
+                           key_bits, block_bits);
     else if (a.lse)
         hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, false, true, WAVES>), grid, block, 0, stream, a, tiles, total,
-                           key_bits, by_item);
+                           key_bits, block_bits);
     else
         hipLaunchKernelGGL((fav4::fwd_kernel_varlen<64, false, false, WAVES>), grid, block, 0, stream, a, tiles, total,
-                           key_bits, by_item);
+                           key_bits, block_bits);
 }
 
 // Checks of the packed-sequence arguments (before any HIP call); the shape
@@ -816,9 +835,9 @@ extern "C" __attribute__((visibility("default"))) int fav4_bshd_forward_varlen(c
         total = std::min(total, a->heads * ((a->total_q + int64_t(a->batch) * (bm - 1)) / bm));
     }
     if (small)
-        launch_varlen<4>(*a, causal, tiles, int(total), key_bits, stream);
+        launch_varlen<4>(*a, causal, tiles, total, key_bits, stream);
     else
-        launch_varlen<8>(*a, causal, tiles, int(total), key_bits, stream);
+        launch_varlen<8>(*a, causal, tiles, total, key_bits, stream);
     return hipGetLastError();
 }
 

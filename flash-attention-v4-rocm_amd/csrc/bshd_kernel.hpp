@@ -154,16 +154,14 @@ __device__ __forceinline__ PackedItem sorted_item(int rank, int batch, int key_b
 // Item id -> (head, rank in the head's item list).  heads a multiple of 8:
 // each XCD (id % 8) works on heads/8 heads, taking their equal ranks side by
 // side, so the query heads of a K/V head share its keys in that XCD's L2;
-// else the heads are dealt round-robin.
-__device__ __forceinline__ void packed_head_rank(int id, int heads, int& head, int& rank) {
-    if ((heads & 7) == 0) {
-        const int per = heads >> 3, slot = id >> 3;
-        rank = slot / per;
-        head = (id & 7) * per + slot - rank * per;
-    } else {
-        rank = id / heads;
-        head = id - rank * heads;
-    }
+// else blocks of 2^block_bits ranks are dealt round-robin, head by head (some
+// ids at the end then have ranks past the list).
+__device__ __forceinline__ void packed_head_rank(int id, int heads, int block_bits, int& head, int& rank) {
+    const bool shares = (heads & 7) == 0;
+    const int slot = id >> 3, j = shares ? slot : (slot >> block_bits) * 8 + (id & 7);
+    const int per = shares ? heads >> 3 : heads, row = j / per, rest = j - row * per;
+    head = shares ? (id & 7) * per + rest : rest;
+    rank = shares ? row : (row << block_bits) + (slot & ((1 << block_bits) - 1));
 }
 
 // Items of a packed batch too large for the lists: `units` for every
@@ -1409,7 +1407,7 @@ void fwd_kernel_chunk(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
         span = {a.sq, a.sk, int64_t(batch) * a.sq, int64_t(batch) * a.sk};
     } else if (a.batch <= MAX_SORTED_SEQS) {
         int rank;
-        packed_head_rank(id, a.heads, head, rank);
+        packed_head_rank(id, a.heads, 0, head, rank);
         const PackedItem it = sorted_item<BM, BN>(rank, a.batch, key_bits, lane, [&](int b) {
             const SeqSpan s = seq_span<KV == 2, true>(sp, b, a.sq, a.sk);
             const int nt = (s.sq + BM - 1) / BM, nk = (s.sk + BN - 1) / BN;
@@ -1584,7 +1582,7 @@ void fwd_kernel_chunk(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
 // ---------------------------------------------------------------------------
 template <int BN, bool CAUSAL, bool LSE, int WAVES, bool BR = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, bool by_item) {
+void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, int block_bits) {
     static_assert(!BR || CAUSAL, "bottom-right is a causal mask");
     constexpr int BM = WAVES * 32;
     constexpr int TILE_BYTES = BN * ROW_BYTES;
@@ -1616,8 +1614,8 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
     };
     // Item order, with key_bits (up to MAX_SORTED_SEQS sequences, unless there is
     // nothing to sort): sorted_item's lists.  A q
-    // tile weighs its key tiles (by_item: with few items per workgroup slot,
-    // where the last ones decide) or its sequence's longest tile's (its q
+    // tile weighs its own key tiles (block_bits < 0: with few items per workgroup
+    // slot, where the last ones decide) or its sequence's longest tile's (its q
     // tiles then run together, heaviest first, and share its K/V in L2).
     // Else: column_item, within a pair the q tiles last-to-first.
     // The lists against that order (graph-timed, causal): 24 sequences of 64..4096
@@ -1632,13 +1630,13 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, boo
         Span sp;
         if (key_bits > 0) {
             int rank;
-            packed_head_rank(id, a.heads, head, rank);
+            packed_head_rank(id, a.heads, max(0, block_bits), head, rank);
             const PackedItem it = sorted_item<BM, BN>(rank, a.batch, key_bits, lane, [&](int b) {
                 // A q tile's visible keys reach the diagonal of its last row.
                 const Span s = span(b);
                 const int nq = s.qe - s.qs, nk = s.ke - s.ks;
                 return PackedSeq{s, (nq + BM - 1) / BM, CAUSAL && !BR ? min(nq, nk) : nk,
-                                 !CAUSAL || !by_item ? INT_MAX : BR ? nk - nq : 0};
+                                 !CAUSAL || block_bits >= 0 ? INT_MAX : BR ? nk - nq : 0};
             });
             if (it.seq < 0) return;
             batch = it.seq;

@@ -164,3 +164,12 @@ def test_packed_sequences_of_few_q_tiles(gpu_runner):
     print("  packed causal 40 x 300 and 44 x 300", flush=True)
     calls = [_packed(torch, gpu_runner, 16, 16, [300] * n, True) for n in (40, 44)]
     assert _ratio(torch, *calls, calls=50) < 0.97
+
+
+def test_packed_heads_in_no_xcd_shares(gpu_runner):
+    """56 sequences of 148 tokens, dense, with 4 heads: as fast as 28 with 8,
+    each sequence's full and short q tile on the same XCD in both."""
+    import torch
+    print("  packed dense 56 x 148 H4 and 28 x 148 H8", flush=True)
+    calls = [_packed(torch, gpu_runner, h, h, [148] * n, False) for h, n in ((4, 56), (8, 28))]
+    assert _ratio(torch, *calls, calls=50) < 1.1

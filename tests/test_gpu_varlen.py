@@ -210,10 +210,11 @@ def test_varlen_bottom_right_causal(gpu_runner, case):
 # (heads, kv_heads, sequences, longest): batches at the edges of the item
 # lists (one, and either side of 64 and of 256 sequences), heads in whole
 # XCD shares and not, few items per workgroup slot and many, both tile sizes;
-# the last four: short sequences on both sides of what is sorted at all, most
-# of them without a query in one.
+# short sequences on both sides of what is sorted at all, most of them without a
+# query in one; ranks in blocks for heads that are no multiple of 8.
 LIST_CASES = [(1, 1, 1, 300), (3, 1, 63, 300), (8, 8, 64, 130), (16, 2, 65, 700), (8, 2, 255, 260), (16, 4, 256, 300),
-              (5, 5, 257, 200), (32, 4, 40, 1300), (3, 3, 256, 64), (8, 2, 70, 64), (8, 2, 70, 65), (4, 4, 200, -60)]
+              (5, 5, 257, 200), (32, 4, 40, 1300), (3, 3, 256, 64), (8, 2, 70, 64), (8, 2, 70, 65), (4, 4, 200, -60), (5, 5, 120, 600),
+              (12, 4, 190, 300)]
 
 
 @pytest.mark.parametrize("case", LIST_CASES, ids=lambda c: "h%dkv%d_n%d_max%d" % c)
