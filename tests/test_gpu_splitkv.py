@@ -193,15 +193,18 @@ def test_splitkv_gqa(gpu_runner, shape):
                 assert np.array_equal(lse.view(np.int32), lsem.view(np.int32)), (causal, "LSE differs")
 
 
-@pytest.mark.parametrize("shape,chunks", [((5, 32, 8, 1, 4096), 19), ((2, 32, 8, 1, 8192), 32), ((4, 32, 8, 1, 4100), 22), ((13, 8, 8, 4, 2000), 7),
-                                          ((96, 4, 4, 3, 1000), 2), ((3, 16, 8, 1, 90), 1)])
-def test_splitkv_decode_auto_chunks(gpu_runner, shape, chunks):
+# (B, H, KVH, Sq, Sk), the plan's chunks and those that run: fewer in the first four.
+@pytest.mark.parametrize("shape,plan,chunks", [((7, 8, 8, 1, 4000), 14, 13), ((2, 32, 8, 1, 8192), 43, 32),
+                                               ((11, 16, 8, 1, 3000), 9, 8), ((13, 8, 8, 4, 2000), 8, 7),
+                                               ((96, 4, 4, 3, 1000), 2, 2), ((3, 16, 8, 1, 90), 1, 1)])
+def test_splitkv_decode_auto_chunks(gpu_runner, shape, plan, chunks):
     """The chunks that Auto runs of a decode call (at most as many as 768
-    one-wave workgroups, or 512 where that makes 32 of a row), bitwise the
-    explicit count's; the call without a workspace and the packed and paged
-    ones of equal lengths the same."""
+    one-wave workgroups, or 512 where that makes 32 of a row; the plan may have
+    more), bitwise the explicit count's; the call without a workspace and the
+    packed and paged ones of equal lengths the same."""
     import torch
     b, h, kvh, sq, sk = shape
+    assert gpu_runner.splitkv_select(b, h, sq, sk, False, kv_heads=kvh) == plan
     q, k, v = (to_device(x, torch.device("cuda:0")) for x in orc.make_inputs(b, h, sq, sk, "normal", seed=71))
     k, v = (x[:, :, :kvh].contiguous() for x in (k, v))
     print(f"  splitkv decode auto {shape} -> {chunks}", flush=True)

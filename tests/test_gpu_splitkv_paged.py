@@ -227,8 +227,7 @@ def _bottom_right_ref(q, k, v, group):
         return o, lse
     if sq <= sk:
         qp = np.concatenate([np.zeros((sk - sq,) + q.shape[1:], dtype=q.dtype), q])[None]
-        ref, ref_lse = orc.attention_fp64(qp, ke, ve, orc.DEFAULT_SCALE, True)
-        return ref[:, sk - sq:], ref_lse[:, :, sk - sq:]
+        return orc.attention_fp64(qp, ke, ve, orc.DEFAULT_SCALE, True, rows=np.arange(sk - sq, sk))
     ref, ref_lse = orc.attention_fp64(q[sq - sk:][None], ke, ve, orc.DEFAULT_SCALE, True)
     o[:, sq - sk:] = ref
     lse[:, :, sq - sk:] = ref_lse
@@ -304,7 +303,7 @@ def _check_dense(o, lse, q, k, v, cu_q, cu_k, lens, group):
 
 @pytest.mark.parametrize("ps", [64, 256])
 def test_splitkv_paged_prefill(gpu_runner, ps):
-    """Queries longer than 32 over paged caches (the 8-wave shape): dense and
+    """Queries longer than 32 over paged caches: dense and
     bottom-right causal against the FP64 oracle on ragged batches (several q
     tiles, q tiles past short sequences, sq > sk), and a uniform batch bitwise
     the contiguous split-KV at the same chunk count."""
@@ -395,6 +394,17 @@ def test_splitkv_paged_presized_workspace_bottom_right(gpu_runner):
     assert torch.equal(lse.view(torch.int32), lse2.view(torch.int32))
 
 
+def _check_close(o, ref, cu_q, case):
+    """Each sequence's O against another call's, RMS-relative.  Both round to
+    BF16 and round their weights to BF16 against bases of their own; each is
+    0.0020-0.0024 from the FP64 result, so they are up to 0.0034 apart."""
+    for a, b in zip(cu_q[:-1], cu_q[1:]):
+        x, y = o[a:b].double(), ref[a:b].double()
+        if b > a and y.any().item():
+            rel = ((x - y).norm() / y.norm()).item()
+            assert rel <= 0.005, (case, int(a), rel)
+
+
 # (heads, kv_heads, page_size, [(sq, sk), ...]): q tiles that end in one chunk
 # beside q tiles that are merged, sizes at the edges of the 64-key and 128- /
 # 256-row tiles, queries without a visible key, few sequences (sorted item
@@ -412,9 +422,9 @@ PREFILL_CASES = [
 def test_paged_prefill_chunks(gpu_runner, case):
     """Bottom-right prefill over paged caches: in one chunk O is bitwise the
     unsplit packed forward's (a q tile of one chunk writes its own O); with
-    more chunks it is within the reference bar (0.01 + 0.01 |ref|) of it, and
-    bitwise the packed K/V call's where the plans agree; nothing is written
-    past O and LSE."""
+    more chunks it is within the reference bar (0.01 + 0.01 |ref|) of it and
+    close to it relative to each sequence's own size, and bitwise the packed
+    K/V call's where the plans agree; nothing is written past O and LSE."""
     import torch
     h, kvh, ps, lens = case
     q, k, v, kc, vc, cu_q, cu_k, seqlens_k, table = _build(h, kvh, ps, lens, seed=97)
@@ -446,6 +456,7 @@ def test_paged_prefill_chunks(gpu_runner, case):
             assert torch.equal(o.view(torch.int16), whole.view(torch.int16))
         else:
             assert ((o.float() - whole.float()).abs() <= 0.01 + 0.01 * whole.float().abs()).all().item(), splits
+            _check_close(o, whole, cu_q, splits)
         seen = torch.isfinite(whole_lse)
         assert torch.equal(torch.isfinite(lse), seen) and torch.equal(torch.isfinite(lse3), seen)
         assert (lse[seen] - whole_lse[seen]).abs().max().item() <= 2e-4, splits
@@ -518,8 +529,10 @@ RANGE_CASES = [
 def test_ragged_decode_ranges(gpu_runner, case):
     """Auto decode of ragged batches, paged and packed, on a workspace full of
     NaN: within the reference bar (0.01 + 0.01 |ref|, LSE 2e-4) of the same
-    call with an explicit chunk count, rows without a key O = 0 and
-    LSE = -inf, nothing written past O, LSE and the workspace."""
+    call with an explicit chunk count and close to it relative to each
+    sequence's own size, rows without a key O = 0 and LSE = -inf, nothing
+    written past O, LSE and the workspace.  Two query heads of the first and of
+    the last K/V head against the FP64 oracle."""
     import torch
     h, kvh, ps, lens, causal = case
     q, k, v, kc, vc, cu_q, cu_k, seqlens_k, table = _build(h, kvh, ps, lens, seed=131)
@@ -547,9 +560,147 @@ def test_ragged_decode_ranges(gpu_runner, case):
             assert torch.isnan(ob[tq:]).all().item() and torch.isnan(lb[h * tq if with_lse else 0:]).all().item()
             assert torch.isnan(ws[need // 4:]).all().item()
             assert ((o.float() - ref.float()).abs() <= 0.01 + 0.01 * ref.float().abs()).all().item(), (paged, with_lse)
+            _check_close(o, ref, cu_q, (paged, with_lse))
             if with_lse:
+                for kh in sorted({0, kvh - 1}):
+                    first, n = kh * (h // kvh), min(2, h // kvh)
+                    check = _check_bottom_right if causal == 2 else _check_dense
+                    check(o[:, first:first + n], lse[first:first + n], q[:, first:first + n], k[:, kh:kh + 1],
+                          v[:, kh:kh + 1], cu_q, cu_k, lens, n, *([paged] if causal == 2 else []))
                 seen = torch.isfinite(ref_lse)
                 assert torch.equal(torch.isfinite(lse), seen) and torch.isneginf(lse[~seen]).all().item()
                 assert (lse[seen] - ref_lse[seen]).abs().max().item() <= 2e-4, paged
             empty = torch.isneginf(ref_lse).T
             assert (o[empty].float() == 0).all().item()
+
+
+@pytest.mark.parametrize("case", RANGE_CASES, ids=lambda c: "h%dkv%d_p%d_n%d_m%d" % (*c[:3], len(c[3]), c[4]))
+def test_ragged_decode_with_a_wrong_total(gpu_runner, case):
+    """total_k only steers Auto: too small, too large and the most possible, it
+    gives a result close to the explicit chunks' and no write past the workspace
+    that the same total asks for."""
+    import torch
+    h, kvh, ps, lens, causal = case
+    q, k, v, kc, vc, cu_q, cu_k, seqlens_k, table = _build(h, kvh, ps, lens, seed=137)
+    dev = torch.device("cuda:0")
+    qd, kcd, vcd = (to_device(x, dev) for x in (q, kc, vc))
+    cq, sk_d, tb = (torch.from_numpy(x).to(dev) for x in (cu_q, seqlens_k, table))
+    max_q, max_k, tq = max(s for s, _ in lens), max(s for _, s in lens), len(q)
+    most = len(lens) * max_k
+    _, _, ref, ref_lse = _out(torch, dev, tq, h, True)
+    gpu_runner.call_splitkv_paged(qd, kcd, vcd, ref, ref_lse, cq, sk_d, tb, max_q, max_k, 5, total_k=len(k),
+                                  causal=causal)
+    for total in (0, len(k) // 7, len(k) // 2, (len(k) + most) // 2, most - 1, most):
+        print(f"  ragged decode h{h} kv{kvh} n{len(lens)} total {total} of {len(k)}", flush=True)
+        need = gpu_runner.splitkv_paged_workspace_size(len(lens), h, kvh, max_q, max_k, tq, total, ps, table.shape[1],
+                                                       len(kc), 0, causal=causal)
+        ws = torch.full((need // 4 + GUARD,), float("nan"), device=dev, dtype=torch.float32)
+        ob, lb, o, lse = _out(torch, dev, tq, h, True)
+        gpu_runner.call_splitkv_paged(qd, kcd, vcd, o, lse, cq, sk_d, tb, max_q, max_k, 0, workspace=ws[:need // 4],
+                                      total_k=total, causal=causal)
+        torch.cuda.synchronize()
+        for guard in (ob[tq:], lb[h * tq:], ws[need // 4:]):
+            assert torch.isnan(guard).all().item(), total
+        _check_close(o, ref, cu_q, total)
+        seen = torch.isfinite(ref_lse)
+        assert torch.equal(torch.isfinite(lse), seen)
+        assert (lse[seen] - ref_lse[seen]).abs().max().item() <= 2e-4, total
+
+
+def test_paged_decode_keeps_64_tiles_a_chunk(gpu_runner):
+    """Equal lengths whose resident workgroups would take more than 64 key tiles
+    a chunk (B32 H8 Sk10208, 319 tiles, page 32: three chunks): Auto keeps to
+    64, a chunk's page numbers in a wave's lanes, and is bitwise five chunks."""
+    import torch
+    b, h, sk, ps = 32, 8, 10208, 32
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    mk = lambda *s: torch.randn(s, device=dev, dtype=torch.float32, generator=g).to(torch.bfloat16)
+    q, kc, vc = mk(b, h, 128), mk(b * sk // ps, ps, h, 128), mk(b * sk // ps, ps, h, 128)
+    table = torch.randperm(b * sk // ps, device=dev, generator=g).to(torch.int32).view(b, -1)
+    cq = torch.arange(b + 1, device=dev, dtype=torch.int32)
+    keys = torch.full((b,), sk, device=dev, dtype=torch.int32)
+    outs = []
+    for splits in (0, 5):
+        o = torch.full_like(q, float("nan"))
+        lse = torch.full((h, b), float("nan"), device=dev, dtype=torch.float32)
+        gpu_runner.call_splitkv_paged(q, kc, vc, o, lse, cq, keys, table, 1, sk, splits, total_k=b * sk)
+        torch.cuda.synchronize()
+        outs.append((o.view(torch.int16), lse.view(torch.int32)))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    rows = [0, 17, 31]
+    pick = lambda c: to_host_bits(c[table[rows].long()].reshape(len(rows), sk, h, 128))
+    ref, ref_lse = orc.attention_fp64(to_host_bits(q[rows])[:, None], pick(kc), pick(vc), orc.DEFAULT_SCALE, False)
+    got = to_host_bits(outs[0][0].view(torch.bfloat16)[rows])[:, None]
+    e = orc.errors(got, outs[0][1].view(torch.float32)[:, rows].T.cpu().numpy()[:, :, None], ref, ref_lse)
+    assert orc.check_acceptance_tolerance(e) and orc.check_reference_tolerance(e), e
+
+
+def _prefill_tile(h, lens, br, splits, cus=256):
+    """The q tile (128 or 256 rows) that an explicit chunk count of a paged
+    prefill runs with, from the library's cost model."""
+    n, max_q, max_k = len(lens), max(s for s, _ in lens), max(s for _, s in lens)
+    total_q, total_k, ktiles = sum(s for s, _ in lens), sum(s for _, s in lens), -(-max_k // 64)
+    tps = min(64, -(-ktiles // min(splits, ktiles)))
+    mean_q, mean_k = total_q / n, total_k / n
+    uniform = 4 * mean_k >= 3 * max_k
+    mean = max(1.0, mean_k / 64 + 0.5 - (0.5 * mean_q / 64 if br else 0.0))
+
+    def predict(bm):
+        slots = cus if bm == 256 else 2 * cus
+        qtiles = h * n * min(-(-max_q // bm), max(1.0, mean_q / bm + 0.5))
+        chunks = max(1.0, np.ceil(mean / tps - 0.25) if uniform else mean / tps + 0.4)
+        items, rounds = qtiles * chunks, qtiles * chunks / slots
+        alone = 1.1 if bm == 128 else 1.0 if max_q <= 128 else 1.45
+        shared = bm == 128 and items > cus
+        per_tile = 1.5 if shared else alone
+        chunk = 7 + per_tile * min(tps, mean)
+        if rounds <= 1:
+            t = 7 + (chunk - 7) * (1.1 if shared else 1.0)
+        elif uniform:
+            t = chunk * (2.0 if rounds <= 2.02 else rounds + 0.5)
+        else:
+            t = qtiles * (chunks * 7 + per_tile * mean) / slots + 0.5 * (7 + per_tile * min(tps, ktiles))
+        return max(t, 7 + alone * min(tps, ktiles))
+
+    return 256 if predict(256) <= predict(128) else 128
+
+
+# (heads, kv_heads, page_size, [(sq, sk), ...], {chunk count: q tile}): both
+# tiles with several q tiles a sequence, more queries than keys, sequences
+# without keys or queries, q tiles of one chunk beside merged ones; one and four
+# sequences a lane in the sorted lists, and more than those hold.
+TILE_CASES = [
+    (8, 2, 64, [(512, 1500), (512, 900), (512, 40), (512, 512), (0, 100), (512, 0), (500, 700), (257, 1400)],
+     {1: 128, 2: 128, 3: 256, 5: 256}),
+] + [(4, 2, 64, [(200 + 37 * i % 57 if i % 9 else 0, 1 + 61 * i % 500 if i % 7 else 0) for i in range(n)], tiles)
+     for n, tiles in ((64, {1: 128, 3: 256}), (65, {1: 256, 3: 256}), (255, {2: 256}), (256, {2: 256}), (257, {2: 256}))
+] + [(4, 2, 64, [(1 + 37 * i % 140, 1 + 61 * i % 500) for i in range(n)], {2: 128}) for n in (65, 256)]
+
+
+@pytest.mark.parametrize("case", TILE_CASES, ids=lambda c: "h%dkv%d_n%d" % (c[0], c[1], len(c[3])))
+def test_prefill_tiles(gpu_runner, case):
+    """Paged prefill, dense and bottom-right, with the q tile that the chunk
+    count takes, against the FP64 oracle."""
+    import torch
+    h, kvh, ps, lens, tiles = case
+    q, k, v, kc, vc, cu_q, cu_k, seqlens_k, table = _build(h, kvh, ps, lens, seed=151)
+    dev = torch.device("cuda:0")
+    qd, kcd, vcd = (to_device(x, dev) for x in (q, kc, vc))
+    cq, sk_d, tb = (torch.from_numpy(x).to(dev) for x in (cu_q, seqlens_k, table))
+    max_q, max_k, tq = max(s for s, _ in lens), max(s for _, s in lens), len(q)
+    for splits, tile in tiles.items():
+        for causal in (2, 0):
+            print(f"  prefill tiles h{h} kv{kvh} n{len(lens)} splits {splits} causal {causal}", flush=True)
+            if causal:
+                assert _prefill_tile(h, lens, True, splits) == tile, splits
+            ob, lb, o, lse = _out(torch, dev, tq, h, True)
+            gpu_runner.call_splitkv_paged(qd, kcd, vcd, o, lse, cq, sk_d, tb, max_q, max_k, splits, total_k=len(k),
+                                          causal=causal)
+            torch.cuda.synchronize()
+            assert torch.isnan(ob[tq:]).all().item() and torch.isnan(lb[h * tq:]).all().item()
+            if causal:
+                _check_bottom_right(o, lse, q, k, v, cu_q, cu_k, lens, h // kvh, splits)
+            else:
+                _check_dense(o, lse, q, k, v, cu_q, cu_k, lens, h // kvh)
