@@ -580,19 +580,19 @@ SplitPlan packed_decode_run(const Fav4Args& a, int kv_heads, int64_t total_k, co
 //    some CUs have two).
 //  * Lengths near the longest (mean >= 3/4): whole rounds of equal chunks; from
 //    the third on their ends spread and half a round is left over.
-//  * Other lengths: the average load per resident workgroup and half a chunk
-//    (the lists start the long chunks first), and never less than the longest.
+//  * Other lengths: the average load per resident workgroup and a fifth of the
+//    longest chunk (the lists start the long ones first), never less than that.
 //  * Merging writes and reads FP32 partials: 4 x 1024 queries against 4096 keys
 //    H32 217 us in one chunk, 290 in two.
-// Other counts than the plan's must promise 4%, and are not taken where the
-// caller does not know the key total (one less than the most), since the lengths
-// may be anything: 43 of 24..94 queries on 6630..52830 keys H4 640 us in the
-// chunks that equal lengths would want, 556 in the plan's 13.  On 245 other
-// batches the choice is 1.5% behind the fastest of the runs on average (at a
-// given chunk count 0.8%), and 7 are slower by more than 2% than the 256-row
-// chunks of the plan's count that every batch once had, the worst by 17% (1.56x
-// on average).  With 9 + 1.1 or 10 + 1.75 per tile and half a q tile counted for
-// a sequence with fewer queries than one, it was 4.2% behind, the worst 1.8x.
+// Other counts than the plan's are not taken where the caller does not know the
+// key total (one less than the most), since the lengths may be anything: 43 of
+// 24..94 queries on 6630..52830 keys H4 640 us in the chunks that equal lengths
+// would want, 556 in the plan's 13.  On 396 other batches the choice is 1.8%
+// behind the fastest of the runs on average (1.1% at a given chunk count), and 7
+// are slower by more than 2% than the 256-row chunks of the plan's count that
+// every batch once had, the worst by 17% (1.5x on average).  With 9 + 1.1 or 10 +
+// 1.75 per tile and half a q tile counted for a sequence with fewer queries than
+// one, it was 4.3% behind, the worst 1.8x.
 SplitPlan packed_prefill_run(const Fav4Args& a, int64_t total_q, int64_t total_k, bool br, const SplitPlan& p,
                              bool choose) {
     const int ktiles = (a.sk + 63) / 64;
@@ -616,11 +616,11 @@ SplitPlan packed_prefill_run(const Fav4Args& a, int64_t total_q, int64_t total_k
         else if (uniform)
             t = chunk * (rounds <= 2.02 ? 2.0 : rounds + 0.5);
         else
-            t = qtiles * (chunks * fixed + per_tile * mean) / slots + 0.5 * (fixed + per_tile * std::min(tps, ktiles));
+            t = qtiles * (chunks * fixed + per_tile * mean) / slots + 0.2 * (fixed + per_tile * std::min(tps, ktiles));
         t = std::max(t, longest);
         if (splits > 1)
             t += 3.5 + double(total_q) * a.heads * splits * 1040 / 3e6 * (uniform ? 1.0 : std::max(0.3, mean_k / a.sk));
-        return tps == p.tps ? t : 1.04 * t;
+        return t;
     };
     const bool unknown = a.batch > 1 && total_k == int64_t(a.batch) * a.sk - 1;
     const int fewest = choose && !unknown ? 1 : p.splits;

@@ -661,7 +661,7 @@ def _prefill_tile(h, lens, br, splits, cus=256):
         elif uniform:
             t = chunk * (2.0 if rounds <= 2.02 else rounds + 0.5)
         else:
-            t = qtiles * (chunks * 7 + per_tile * mean) / slots + 0.5 * (7 + per_tile * min(tps, ktiles))
+            t = qtiles * (chunks * 7 + per_tile * mean) / slots + 0.2 * (7 + per_tile * min(tps, ktiles))
         return max(t, 7 + alone * min(tps, ktiles))
 
     return 256 if predict(256) <= predict(128) else 128
@@ -675,7 +675,7 @@ TILE_CASES = [
     (8, 2, 64, [(512, 1500), (512, 900), (512, 40), (512, 512), (0, 100), (512, 0), (500, 700), (257, 1400)],
      {1: 128, 2: 128, 3: 256, 5: 256}),
 ] + [(4, 2, 64, [(200 + 37 * i % 57 if i % 9 else 0, 1 + 61 * i % 500 if i % 7 else 0) for i in range(n)], tiles)
-     for n, tiles in ((64, {1: 128, 3: 256}), (65, {1: 256, 3: 256}), (255, {2: 256}), (256, {2: 256}), (257, {2: 256}))
+     for n, tiles in ((64, {1: 128, 3: 256}), (65, {1: 128, 3: 256}), (255, {2: 256}), (256, {2: 256}), (257, {2: 256}))
 ] + [(4, 2, 64, [(1 + 37 * i % 140, 1 + 61 * i % 500) for i in range(n)], {2: 128}) for n in (65, 256)]
 
 
