@@ -14,7 +14,8 @@
 
 namespace {
 
-// Upper bound on launched workgroups; larger problems loop inside the kernel.
+// Most workgroups in a grid dimension.  Larger decode chunk and merge grids loop
+// inside the kernel, the other kernels take a second dimension (item_grid).
 constexpr int64_t MAX_GRID = int64_t(1) << 22;
 
 // CU count of the current device (256 if it cannot be read), cached per
@@ -43,8 +44,8 @@ int launch(const Fav4Args& a, const fav4::Layout& L, hipStream_t stream) {
     const int tiles = (a.sq + BM - 1) / BM;
     const int64_t bh = int64_t(a.batch) * a.heads;
     // Causal q tiles go in pairs of equal cost unless each has a CU of its own
-    // (B3 H5 S1500, 180 q tiles: 33.8 us paired, 29.4 not; B4 H16 S2048, 1024
-    // q tiles: 82 and 113).
+    // (B3 H5 S1500, 180 q tiles: 33.8 us paired, 29.4 not; B4 H16 S2048 in
+    // config 1, 1024 q tiles: 82 and 113).
     const bool paired = CAUSAL && bh * tiles > device_cus();
     const int64_t total = bh * fav4::items_per_head(tiles, paired);
     if (total > INT_MAX) return hipErrorInvalidValue;
@@ -140,12 +141,17 @@ struct SplitPlan {
 
 // Auto for prefill (Sq > 32).  Filling the CUs is not enough: on the small
 // grids where splitting is considered, the unsplit forward runs 128-row q
-// tiles two per CU (causal: a heavy tile paired with a light one), while the
-// split kernel runs 256-row (q tile, chunk) items one per CU with higher fixed
-// costs.  Auto therefore keeps, among 1..max_splits chunks, the count with
-// the lowest predicted time.  The model (microseconds; fitted to graph-timed
-// MI355X runs of 23 shapes, B1-4, H1-64, Sq 256-16384, Sk up to 65536, where
-// it picks the fastest measured choice or one within 2% of it):
+// tiles two per CU, while the split kernel runs 256-row (q tile, chunk) items
+// one per CU with higher fixed costs.  Auto therefore keeps, among
+// 1..max_splits chunks, the count with the lowest predicted time.  The model
+// (microseconds) was fitted to graph-timed MI355X runs of 23 shapes (B1-4, H1-64,
+// Sq 256-16384, Sk up to 65536) with earlier kernels, whose causal forward
+// always paired a heavy q tile with a light one and whose packed forward
+// launched every q tile up to the longest sequence.  With the present ones, on
+// 70 random shapes of that range, its choice is 4.7% behind the fastest
+// measured on average: 49 shapes within 2%, 13 over 10%, the worst 1.5x (B4 H1
+// 510 x 1495 dense unsplit 29.6 us, in 6 chunks 19.5), none slower than with the
+// kernels that it was fitted to by more than 3%:
 //  * unsplit: rounds * (9 + c per 64-key tile of an item), an item being a
 //    q tile (dense; c = 0.9 with at most one workgroup per CU, else 1.0) or
 //    the heaviest tile pair (causal; c = 1.0);
@@ -536,18 +542,19 @@ SplitPlan packed_split_plan(const Fav4Args& a, int kv_heads, int64_t total_k, in
 // one-wave workgroups per CU (fwd_kernel_ranges), unless
 //  * every sequence has the longest one's keys (the contiguous call's chunks
 //    then, and its result bitwise);
-//  * a range would be under MIN_RANGE_TILES key tiles: the short ranges' fixed
-//    cost then outweighs their balance (H32 KVH8, plan / ranges: 8.5 tiles, 32
-//    sequences of 64..2048 keys 28.5 / 26.2 us; 4.1 tiles, 3 of 2500..3000
-//    15.6 / 17.3; 2.5 tiles, 8 of 100..2000 15.0 / 16.4);
+//  * a range would be under MIN_RANGE_TILES key tiles, not counting its
+//    sequences' own cost: the short ranges then gain nothing or lose (plan /
+//    ranges, H32 KVH8: 10 tiles, 32 sequences of 64..2048 keys 28.6 / 22.7 us;
+//    4.2 tiles, 3 of 2500..3000 14.1 / 14.0; 2.6 tiles, 8 of 100..2000 14.2 both;
+//    0.3 - 1.4 tiles, 24 - 84 sequences of 30..110 9.5 - 12.9 / 11.3 - 14.2);
 //  * the plan's chunks would not hold the ranges: a sequence of n tiles meets
 //    at most (n - 2) / (range length) + 2 of them, so `splits` chunks suffice
 //    for ranges of at least ktiles / (splits - 1) tiles, which the kernel keeps
 //    to;
 //  * the batch has more sequences than a wave's lanes list.
 // Two workgroups per CU against three (the plan's): 32 sequences of 1k..32k
-// keys 207 and 210 us, 64 of 64..2048 38 and 41, 200 of 300..9000 337 and 341,
-// 16 of 8 queries H64 on 1k..16k 102 and 115; 8 of 1k..32k 87 and 86.
+// keys 202 us both, 64 of 64..2048 40.9 and 41.5, 200 of 300..9000 346 and 349,
+// 16 of 8 queries H64 on 1k..16k 121 and 130, 8 of 1k..32k 93 and 121.
 constexpr int RANGE_WGS_PER_CU = 2;
 constexpr int MIN_RANGE_TILES = 8;
 SplitPlan packed_decode_run(const Fav4Args& a, int kv_heads, int64_t total_k, const SplitPlan& p,
@@ -673,8 +680,8 @@ int64_t varlen_workspace(const Fav4VarlenArgs& v, const SplitPlan& p, int causal
 constexpr int PAGED_MAX_TPS = 64;          // key tiles per chunk: one page number per lane
 constexpr int PAGED_MAX_KEYS = fav4::MAX_SPLITS * PAGED_MAX_TPS * 32;
 
-// Decode (max_seqlen_q <= 32) needs page_size % 32 == 0 (one 32-key tile per
-// page), prefill page_size % 64 == 0 (the 8-wave shape's 64-key tiles).
+// Decode (max_seqlen_q <= 32) needs page_size % 32 == 0 (a 32-key tile lies in
+// one page), prefill page_size % 64 == 0 (64-key tiles).
 int paged_shape_ok(const Fav4PagedArgs* a, int causal, int splits) {
     if (!a || a->batch <= 0 || a->heads <= 0 || a->kv_heads <= 0 || a->heads % a->kv_heads != 0 ||
         a->max_seqlen_q <= 0 || a->max_seqlen_q > MAX_SPLIT_SQ || a->max_seqlen_k <= 0 || a->total_q <= 0 ||
@@ -715,8 +722,10 @@ Fav4Args paged_shape(const Fav4PagedArgs& v) {
     return a;
 }
 
-// The packed-batch plan, with chunks capped at 64 key tiles (a chunk's page
-// numbers fit the lanes of one wave); one chunk still runs the split kernels.
+// The packed-batch plan, with chunks capped at 64 key tiles (a decode chunk's
+// page numbers fit the lanes of one wave; the prefill chunks and the ranges,
+// which may be longer, load them 64 at a time); one chunk still runs the split
+// kernels.
 SplitPlan paged_plan(const Fav4PagedArgs& v, int causal, int req) {
     const Fav4Args a = paged_shape(v);
     // Prefill: the contiguous prefill plan at the max lengths (bottom-right

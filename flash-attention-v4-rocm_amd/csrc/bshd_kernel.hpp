@@ -512,9 +512,10 @@ __device__ __forceinline__ void pv_plain(const unsigned char* vs, const LdsOffse
 //  * Rows r >= rows (past the sequence) store nothing: their 32-bit offsets
 //    could wrap into a valid row for large row strides.
 //  * LANE_OPAQUE derives the lane offsets from an opaque copy of the lane
-//    id, so that the compiler does not hoist them out of the item loop and
-//    keep them live through the key loop (where the LSE kernels' register
-//    budget is tight; hoisted, causal LSE spilled).
+//    id, so that the compiler does not compute them before the key loop and
+//    keep them live through it (the causal LSE kernels, which loop over a pair
+//    of q tiles, take 236 and 232 VGPRs with it and 255 without, the other LSE
+//    kernels 1-6 more).
 template <int TILE_BYTES, bool LANE_OPAQUE>
 __device__ __forceinline__ void store_o_rows(const RowState& st, float inv, unsigned char* smem, uint32_t slot,
                                              rsrc_t ro, uint32_t orow, int wrow0, int rows, int lane) {
@@ -842,9 +843,9 @@ void fwd_kernel(Fav4Args a, Layout L, int tiles, int total, bool paired) {
 // ---------------------------------------------------------------------------
 // Split-KV: the key range of every (batch, head, q tile) is cut into `splits`
 // chunks of `tps` key tiles, each chunk is attended by its own workgroup (same
-// tile body as fwd_kernel, 3 LDS stages), and a second kernel merges the
-// chunks.  For few (b, h, q tile) items and long
-// keys this fills the GPU where one workgroup per item cannot.
+// tile body as fwd_kernel), and a second kernel merges the chunks.  For few
+// (b, h, q tile) items and long keys this fills the GPU where one workgroup per
+// item cannot.
 // Workspace (FP32, caller-owned):
 //   o_part  [splits][B*H][sq][128]  O of the chunk, normalised by its own
 //                                    BF16 weight sum lb_s
@@ -1119,9 +1120,9 @@ void fwd_kernel_split(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
 // workgroup: chunks cut per sequence (4096 of up to 64 tiles for the batch
 // below, two thirds of them past their sequence's keys) left the last round of
 // resident workgroups mostly idle.  32 sequences of 1k..32k keys H32 KVH8 (1.28
-// GB) 255 -> 207 us with the merge, 5.0 -> 6.2 TB/s; 8 of them 110 -> 87; 32 of
-// 6000..8192 keys 201 -> 147; 16 of 8 queries H64 KVH8 on 1k..16k 135 -> 102.
-// A fourth LDS stage (three tiles in flight) gives nothing (209 us).
+// GB) 260 -> 202 us with the merge, 4.9 -> 6.4 TB/s; 8 of them 126 -> 93; 32 of
+// 6000..8192 keys 203 -> 157; 16 of 8 queries H64 KVH8 on 1k..16k 184 -> 120.
+// A fourth LDS stage (three tiles in flight) gave nothing (209 us against 207).
 //  * tiles: 32-row q tiles of a group's row space; ranges: workgroups per
 //    (K/V head, q tile), all of them resident at once; min_tiles: the range
 //    length below which the longest sequence could meet more than sp.splits
@@ -1572,10 +1573,11 @@ void fwd_kernel_chunk(Fav4Args a, SplitArgs sp, int kv_heads, int tiles, int tot
 // Varlen: packed sequences.  Q/O are [total_q, heads, 128] and K/V
 // [total_k, kv_heads, 128]; sequence b owns rows [cu_seqlens_q[b],
 // cu_seqlens_q[b+1]) and [cu_seqlens_k[b], cu_seqlens_k[b+1]); LSE is
-// [heads, total_q].  One item per (b, h, 256-row
-// q tile up to max_seqlen_q); items past a sequence's end do nothing.  The
-// offsets read from device memory are clamped to [0, total] and to the
-// maximum lengths, so every access stays inside the caller's buffers.
+// [heads, total_q].  One workgroup per (b, h, 128- or 256-row q tile): of those
+// that exist in the sorted lists' order, else of all up to max_seqlen_q, where
+// the ones past a sequence's end do nothing.  The offsets read from device
+// memory are clamped to [0, total] and to the maximum lengths, so every access
+// stays inside the caller's buffers.
 // BR (with CAUSAL): bottom-right causal, query i of a sequence with sq queries
 // and sk keys sees keys j <= sk - sq + i; with sq > sk the first sq - sk rows
 // see none and give O = 0, LSE = -inf.
@@ -1622,135 +1624,131 @@ void fwd_kernel_varlen(Fav4VarlenArgs a, int tiles, int total, int key_bits, int
     // tokens H32 KVH8 708 -> 582 us, 64 of 100..1000 H8 69 -> 55, 4 x 2048
     // H16 105 -> 77 (by sequence 97), 8 x 4096 H8 313 -> 264 (313); 32 of
     // 1024..7168 H8 858 -> 848.
-    {
-        const uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;
-        if (wg >= uint32_t(total)) return;
-        const int id = int(wg);
-        int batch, head, tile;
-        Span sp;
-        if (key_bits > 0) {
-            int rank;
-            packed_head_rank(id, a.heads, max(0, block_bits), head, rank);
-            const PackedItem it = sorted_item<BM, BN>(rank, a.batch, key_bits, lane, [&](int b) {
-                // A q tile's visible keys reach the diagonal of its last row.
-                const Span s = span(b);
-                const int nq = s.qe - s.qs, nk = s.ke - s.ks;
-                return PackedSeq{s, (nq + BM - 1) / BM, CAUSAL && !BR ? min(nq, nk) : nk,
-                                 !CAUSAL || block_bits >= 0 ? INT_MAX : BR ? nk - nq : 0};
-            });
-            if (it.seq < 0) return;
-            batch = it.seq;
-            sp = it.span;
-            tile = (sp.qe - sp.qs + BM - 1) / BM - 1 - it.place;       // from the last q tile down
-        } else {
-            int unit;
-            column_item(id, total, a.batch, a.heads, tiles, batch, head, unit);
-            tile = tiles - 1 - unit;
-            sp = span(batch);
+    const uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;
+    if (wg >= uint32_t(total)) return;
+    const int id = int(wg);
+    int batch, head, tile;
+    Span sp;
+    if (key_bits > 0) {
+        int rank;
+        packed_head_rank(id, a.heads, max(0, block_bits), head, rank);
+        const PackedItem it = sorted_item<BM, BN>(rank, a.batch, key_bits, lane, [&](int b) {
+            // A q tile's visible keys reach the diagonal of its last row.
+            const Span s = span(b);
+            const int nq = s.qe - s.qs, nk = s.ke - s.ks;
+            return PackedSeq{s, (nq + BM - 1) / BM, CAUSAL && !BR ? min(nq, nk) : nk,
+                             !CAUSAL || block_bits >= 0 ? INT_MAX : BR ? nk - nq : 0};
+        });
+        if (it.seq < 0) return;
+        batch = it.seq;
+        sp = it.span;
+        tile = (sp.qe - sp.qs + BM - 1) / BM - 1 - it.place;       // from the last q tile down
+    } else {
+        int unit;
+        column_item(id, total, a.batch, a.heads, tiles, batch, head, unit);
+        tile = tiles - 1 - unit;
+        sp = span(batch);
+    }
+    batch = __builtin_amdgcn_readfirstlane(batch);
+    head = __builtin_amdgcn_readfirstlane(head);
+    tile = __builtin_amdgcn_readfirstlane(tile);
+    const int qs = __builtin_amdgcn_readfirstlane(sp.qs), ks = __builtin_amdgcn_readfirstlane(sp.ks);
+    const int sq = __builtin_amdgcn_readfirstlane(sp.qe) - qs, sk = __builtin_amdgcn_readfirstlane(sp.ke) - ks;
+    const int q0 = tile * BM;
+    if (q0 >= sq) return;    // uniform over the workgroup
+    const int qw = q0 + wave * 32, row = qw + col;
+    const int64_t qrow0 = (int64_t(qs) + q0) * a.heads + head;
+    const int64_t krow0 = int64_t(ks) * a.kv_heads + head / group;
+    const char* kbase = static_cast<const char*>(a.k) + krow0 * ROW_BYTES;
+    const char* vbase = static_cast<const char*>(a.v) + krow0 * ROW_BYTES;
+    const rsrc_t rq = make_rsrc(static_cast<const char*>(a.q) + qrow0 * ROW_BYTES,
+                                uint32_t(sq - q0 - 1) * row_bytes + ROW_BYTES);
+    const rsrc_t ro = make_rsrc(static_cast<char*>(a.o) + qrow0 * ROW_BYTES,
+                                uint32_t(sq - q0 - 1) * row_bytes + ROW_BYTES);
+    // Key tiles [0, nfull) are unmasked for every row of the q tile;
+    // BR: up to the last row's diagonal, and unmasked below the first
+    // row's (shift = sk - sq; may be negative).
+    const int shift = BR ? sk - sq : 0;
+    const int kend = !CAUSAL ? sk : BR ? min(sk, max(0, min(sq, q0 + BM) + shift)) : min(sk, q0 + BM);
+    const int ntiles = (kend + BN - 1) / BN;
+    const int nfull = (!CAUSAL ? sk : BR ? max(0, min(sk, q0 + 1 + shift)) : min(sk, q0 + 1)) / BN;
+    const int climit = row + shift;    // last visible key of this lane's row (causal)
+
+    RowState st;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) st.o[db] = f32x16{};
+    st.m = -__builtin_inff();
+    st.lb = 0.f;
+    st.l = 0.f;
+
+    if (ntiles > 0) {
+        auto issue = [&](int t) {
+            const int64_t first = int64_t(t) * BN;
+            const uint32_t bytes = uint32_t(sk - int(first) - 1) * kv_row_bytes + ROW_BYTES;
+            const u32x4 rk = make_desc(kbase + first * kv_row_bytes, bytes);
+            const u32x4 rv = make_desc(vbase + first * kv_row_bytes, bytes);
+            dma_tile<DMA, TILE_BYTES>(rk, rv, smem_base + (t & 1) * STAGE_BYTES, wave, dofs);
+        };
+        issue(0);
+        bf16x8 qr[8];
+        {
+            const uint32_t qoff = uint32_t(wave * 32 + col) * row_bytes + half * 16;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) qr[c] = load16(rq, qoff + c * 32);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) asm volatile("" ::"v"(qr[c]));
         }
-        batch = __builtin_amdgcn_readfirstlane(batch);
-        head = __builtin_amdgcn_readfirstlane(head);
-        tile = __builtin_amdgcn_readfirstlane(tile);
-        const int qs = __builtin_amdgcn_readfirstlane(sp.qs), ks = __builtin_amdgcn_readfirstlane(sp.ks);
-        const int sq = __builtin_amdgcn_readfirstlane(sp.qe) - qs, sk = __builtin_amdgcn_readfirstlane(sp.ke) - ks;
-        const int q0 = tile * BM;
-        if (q0 >= sq) return;    // uniform over the workgroup
-        const int qw = q0 + wave * 32, row = qw + col;
-        const int64_t qrow0 = (int64_t(qs) + q0) * a.heads + head;
-        const int64_t krow0 = int64_t(ks) * a.kv_heads + head / group;
-        const char* kbase = static_cast<const char*>(a.k) + krow0 * ROW_BYTES;
-        const char* vbase = static_cast<const char*>(a.v) + krow0 * ROW_BYTES;
-        const rsrc_t rq = make_rsrc(static_cast<const char*>(a.q) + qrow0 * ROW_BYTES,
-                                    uint32_t(sq - q0 - 1) * row_bytes + ROW_BYTES);
-        const rsrc_t ro = make_rsrc(static_cast<char*>(a.o) + qrow0 * ROW_BYTES,
-                                    uint32_t(sq - q0 - 1) * row_bytes + ROW_BYTES);
-        // Key tiles [0, nfull) are unmasked for every row of the q tile;
-        // BR: up to the last row's diagonal, and unmasked below the first
-        // row's (shift = sk - sq; may be negative).
-        const int shift = BR ? sk - sq : 0;
-        const int kend = !CAUSAL ? sk : BR ? min(sk, max(0, min(sq, q0 + BM) + shift)) : min(sk, q0 + BM);
-        const int ntiles = (kend + BN - 1) / BN;
-        const int nfull = (!CAUSAL ? sk : BR ? max(0, min(sk, q0 + 1 + shift)) : min(sk, q0 + 1)) / BN;
-        const int climit = row + shift;    // last visible key of this lane's row (causal)
-
-        RowState st;
-#pragma unroll
-        for (int db = 0; db < 4; ++db) st.o[db] = f32x16{};
-        st.m = -__builtin_inff();
-        st.lb = 0.f;
-        st.l = 0.f;
-
-        if (ntiles > 0) {
-            auto issue = [&](int t) {
-                const int64_t first = int64_t(t) * BN;
-                const uint32_t bytes = uint32_t(sk - int(first) - 1) * kv_row_bytes + ROW_BYTES;
-                const u32x4 rk = make_desc(kbase + first * kv_row_bytes, bytes);
-                const u32x4 rv = make_desc(vbase + first * kv_row_bytes, bytes);
-                dma_tile<DMA, TILE_BYTES>(rk, rv, smem_base + (t & 1) * STAGE_BYTES, wave, dofs);
-            };
-            issue(0);
-            bf16x8 qr[8];
-            {
-                const uint32_t qoff = uint32_t(wave * 32 + col) * row_bytes + half * 16;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) qr[c] = load16(rq, qoff + c * 32);
-#pragma unroll
-                for (int c = 0; c < 8; ++c) asm volatile("" ::"v"(qr[c]));
-            }
-            auto step = [&](auto stage_c, auto masked_c, int t) {
-                constexpr int STAGE = decltype(stage_c)::value;
-                const unsigned char* cur = smem + STAGE * STAGE_BYTES;
+        auto step = [&](auto stage_c, auto masked_c, int t) {
+            constexpr int STAGE = decltype(stage_c)::value;
+            const unsigned char* cur = smem + STAGE * STAGE_BYTES;
+            wait_vmem();
+            __syncthreads();
+            if (t + 1 < ntiles) issue(t + 1);
+            // A causal tile entirely above this wave's rows changes nothing.
+            // BR rows that see no key yet keep a -inf base (EMPTY).
+            if (!(decltype(masked_c)::value && CAUSAL) || t * BN <= qw + 31 + shift)
+                attend_fused<BN, decltype(masked_c)::value, CAUSAL, LSE, BR>(
+                    cur, cur + TILE_BYTES, off, qr, st, t == 0, t * BN, sk, climit, half, scale2);
+        };
+        using S0 = std::integral_constant<int, 0>;
+        using S1 = std::integral_constant<int, 1>;
+        using Plain = std::integral_constant<bool, false>;
+        using Masked = std::integral_constant<bool, true>;
+        int t = 0;
+        if (qw >= sq) {
+            // Rows all past this sequence's end: only the DMA and barrier
+            // sequence of the loop below.
+            for (; t < ntiles; ++t) {
                 wait_vmem();
                 __syncthreads();
                 if (t + 1 < ntiles) issue(t + 1);
-                // A causal tile entirely above this wave's rows changes nothing.
-                // BR rows that see no key yet keep a -inf base (EMPTY).
-                if (!(decltype(masked_c)::value && CAUSAL) || t * BN <= qw + 31 + shift)
-                    attend_fused<BN, decltype(masked_c)::value, CAUSAL, LSE, BR>(
-                        cur, cur + TILE_BYTES, off, qr, st, t == 0, t * BN, sk, climit, half, scale2);
-            };
-            using S0 = std::integral_constant<int, 0>;
-            using S1 = std::integral_constant<int, 1>;
-            using Plain = std::integral_constant<bool, false>;
-            using Masked = std::integral_constant<bool, true>;
-            int t = 0;
-            if (qw >= sq) {
-                // Rows all past this sequence's end: only the DMA and barrier
-                // sequence of the loop below.
-                for (; t < ntiles; ++t) {
-                    wait_vmem();
-                    __syncthreads();
-                    if (t + 1 < ntiles) issue(t + 1);
-                }
-            } else {
-                for (; t + 1 < nfull; t += 2) {
-                    step(S0{}, Plain{}, t);
-                    step(S1{}, Plain{}, t + 1);
-                }
-                // Masked tiles in compile-time stage pairs too (t is even):
-                // no runtime choice of step body, so O keeps one home.
-                for (; t + 1 < ntiles; t += 2) {
-                    step(S0{}, Masked{}, t);
-                    step(S1{}, Masked{}, t + 1);
-                }
-                if (t < ntiles) step(S0{}, Masked{}, t);
             }
+        } else {
+            for (; t + 1 < nfull; t += 2) {
+                step(S0{}, Plain{}, t);
+                step(S1{}, Plain{}, t + 1);
+            }
+            // Masked tiles in compile-time stage pairs too (t is even):
+            // no runtime choice of step body, so O keeps one home.
+            for (; t + 1 < ntiles; t += 2) {
+                step(S0{}, Masked{}, t);
+                step(S1{}, Masked{}, t + 1);
+            }
+            if (t < ntiles) step(S0{}, Masked{}, t);
         }
+    }
 
-        // O = acc / lb (0 for a sequence without keys), BF16.  Rows past the
-        // sequence store nothing (their 32-bit offsets can wrap into a valid
-        // row when heads * 256 bytes is large).
-        const float inv = st.lb > 0.f ? 1.f / st.lb : 0.f;
-        // Stage ntiles % 2 receives no DMA in this q tile and its last tile
-        // (ntiles - 2) was read before the last step's barrier (with fewer
-        // tiles it was never used, and the previous q tile's final wait and
-        // barrier retired everything): this wave's slots there hold the O
-        // staging.
-        store_o_rows<TILE_BYTES, LSE>(st, inv, smem, uint32_t((ntiles & 1) * STAGE_BYTES + wave * DMA * 1024), ro,
-                                      row_bytes, wave * 32, sq - qw, lane);
-        if constexpr (LSE) {
-            if (half == 0 && row < sq) a.lse[int64_t(head) * a.total_q + qs + row] = __builtin_fmaf(st.m, LN2, logf(st.l));
-        }
+    // O = acc / lb (0 for a sequence without keys), BF16.  Rows past the
+    // sequence store nothing (their 32-bit offsets can wrap into a valid
+    // row when heads * 256 bytes is large).
+    const float inv = st.lb > 0.f ? 1.f / st.lb : 0.f;
+    // Stage ntiles % 2 receives no DMA after tile ntiles - 2's, which was
+    // read before the last step's barrier (with one tile or none that stage
+    // was never used): this wave's slots there hold the O staging.
+    store_o_rows<TILE_BYTES, LSE>(st, inv, smem, uint32_t((ntiles & 1) * STAGE_BYTES + wave * DMA * 1024), ro,
+                                  row_bytes, wave * 32, sq - qw, lane);
+    if constexpr (LSE) {
+        if (half == 0 && row < sq) a.lse[int64_t(head) * a.total_q + qs + row] = __builtin_fmaf(st.m, LN2, logf(st.l));
     }
 }
 
@@ -1846,8 +1844,8 @@ __global__ __launch_bounds__(256) void combine_kernel(Fav4Args a, SplitArgs sp) 
         if (live) {
 #pragma unroll
             for (int i = 0; i < NS; ++i) {
-                const int s = part + i * PER;
-                if (s < sp.splits) xo[i] = *reinterpret_cast<const f32x4*>(op + (DECODE ? s : min(s, nch - 1)) * slab * D);
+                const int s = part + i * PER, row = DECODE ? s : min(s, nch - 1);
+                if (s < sp.splits) xo[i] = *reinterpret_cast<const f32x4*>(op + row * slab * D);
             }
         }
         float vb = -__builtin_inff(), vl = -__builtin_inff();
