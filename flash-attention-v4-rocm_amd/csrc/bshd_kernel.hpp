@@ -287,12 +287,15 @@ __device__ __forceinline__ void dma_tile(u32x4 rk, u32x4 rv, uint32_t stage, int
 // barriers hold that order: left alone, the compiler picks it or a chain per
 // block with the register pressure around it, and the chain is 2-4% slower
 // (packed 8 x 4096 H32 causal 1069 us against 1028; three or all eight chunks
-// ahead lose again on the dense forward).
+// ahead lose again on the dense forward).  With the LSE the last MFMAs may mix
+// with the softmax, whose additional sums there then start earlier: dense B1 H8
+// S5000 147 -> 143 us, S4096 79.4 -> 77.1, within 1% elsewhere; without it
+// dense B32 H8 S4096 goes 1911 -> 1933.
 // Masked tiles compute every block too (no branch around blocks past the key
 // length or above the diagonal): tile_mask then hides them, and the tile
 // stays one basic block for the scheduler.  K rows past sk hold zeros (the
 // DMA's bounded buffer returns 0 there), so those scores are finite.
-template <int BN>
+template <int BN, bool LSE = false>
 __device__ __forceinline__ void tile_qk(const unsigned char* ks, const LdsOffsets& off, const bf16x8 (&qr)[8],
                                         f32x16 (&s)[BN / 32]) {
     constexpr int KB = BN / 32;
@@ -310,7 +313,7 @@ __device__ __forceinline__ void tile_qk(const unsigned char* ks, const LdsOffset
         if (c + 2 < 8) read(c + 2);
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) s[kb] = mfma32(kop[c][kb], qr[c], c ? s[kb] : zero);
-        __builtin_amdgcn_sched_barrier(0);
+        if (!LSE || c < 7) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -449,7 +452,7 @@ __device__ __forceinline__ void attend_fused(const unsigned char* ks, const unsi
                                              int row, int half, float scale2) {
     f32x16 s[BN / 32];
     __builtin_amdgcn_s_setprio(1);
-    tile_qk<BN>(ks, off, qr, s);
+    tile_qk<BN, LSE>(ks, off, qr, s);
     __builtin_amdgcn_s_setprio(0);
     attend_tail<BN, MASKED, CAUSAL, LSE, EMPTY>(s, vs, off, st, first, start, sk, row, half, scale2);
 }
